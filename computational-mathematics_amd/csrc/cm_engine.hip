@@ -46,6 +46,7 @@
 #include "cm_solve.h"
 #include "cm_batch.hpp"
 #include "cm_block.hpp"
+#include "cm_resident.hpp"
 #include "cm_trsv.hpp"
 #include "cm_pdfiim.hpp"
 
@@ -302,6 +303,7 @@ struct SlotIndex {
 struct DiaIndex {
     int n = 0, ldn = 0, nd = 0;  // ldn: diagonal stride, n rounded up to DIA_ALIGN
     long long nrem = 0;
+    std::vector<int> hoff;  // the offsets on the host, ascending
     int *off = nullptr, *dsrc = nullptr, *rptr = nullptr, *rcol = nullptr, *rsrc = nullptr;
     // Rows whose remainder is longer than SHORT_MAX, for the block products:
     // lpos[row] = their index q (0..nlong-1), -1 for the other rows.  Their
@@ -784,6 +786,7 @@ static int build_dia_device(DevCsr<double> &m, hipStream_t s, bool *done)
     D->n = n;
     D->ldn = ldn;
     D->nd = nd;
+    D->hoff = off;
     CM_TRY(dev_upload(&D->off, off.data(), off.size(), s));
     // positions on the selected diagonals (map: offset -> diagonal), remainder counts
     k_fill_int<<<long_grid((long long)nmap), BS, 0, s>>>((long long)nmap, -1, map);
@@ -863,6 +866,7 @@ static int build_dia(DevCsr<double> &m, hipStream_t s)
         CM_TRY(dev_upload(&D->lcol, L.lcol.data(), L.lcol.size(), s));
         CM_TRY(dev_upload(&D->lsrc, L.lsrc.data(), L.lsrc.size(), s));
     }
+    D->hoff = L.off;
     CM_TRY(dev_upload(&D->off, L.off.data(), L.off.size(), s));
     CM_TRY(dev_upload(&D->dsrc, L.dsrc.data(), L.dsrc.size(), s));
     if (D->nrem) {
@@ -1101,6 +1105,10 @@ struct Krylov {
     // when no launch is being bracketed by profiling events
     bool use_graph = true;
     hipGraphExec_t g1 = nullptr, gN = nullptr;
+    bool resident = false;       // whole solves in one launch (tuned systems; run_resident)
+    double *rs_slots = nullptr;  // reduction slots and control words of the resident solve (first use)
+    RsCtl *rs_ctl = nullptr;
+    RsArgs<T, VA, VF> *rs_args = nullptr;
 
     void drop_graphs()
     {
@@ -1117,6 +1125,9 @@ struct Krylov {
         for (T *q : bufs) (void)hipFree(q);
         (void)hipFree(partials);
         (void)hipFree(trace);
+        (void)hipFree(rs_slots);
+        (void)hipFree(rs_ctl);
+        (void)hipFree(rs_args);
         (void)hipFree(st);
         if (hst) (void)hipHostFree(hst);
         for (auto &e : ev)
@@ -1473,8 +1484,7 @@ struct Krylov {
         return CM_OK;
     }
 
-    // Writes the initial state (done = 0) of a solve of NMAX passes.
-    int begin(double tol, int NMAX, int info_in, int trace_cap)
+    int ensure_trace(int trace_cap)
     {
         if (trace_cap > 0 && trace_cap > trace_cap_dev) {
             (void)hipFree(trace);
@@ -1482,6 +1492,104 @@ struct Krylov {
             CM_HIP(hipMalloc((void **)&trace, (size_t)trace_cap * sizeof(double)));
             trace_cap_dev = trace_cap;
         }
+        return CM_OK;
+    }
+
+    // Matrix m for workgroups of `rows` rows, bsz of them per step: its
+    // diagonal copy where that is built (whichever format the launched
+    // products use) and its x windows fit, else CSR.
+    template <class V>
+    static RsMat<V> rs_mat(const DevCsr<V> &m, int bsz, int rows)
+    {
+        RsMat<V> q;
+        std::memset(&q, 0, sizeof q);
+        q.rowscale = m.rowscale;
+        if (m.dia && m.dval && rs_windows(m.dia->hoff, bsz, rows, q)) {
+            const DiaIndex &D = *m.dia;
+            q.nd = D.nd;
+            q.ldn = D.ldn;
+            q.dval = m.dval;
+            q.ptr = D.rptr;
+            q.col = D.rcol;
+            q.val = m.rval;
+        } else {
+            q.ns = 0;
+            q.ptr = m.ptr;
+            q.col = m.col;
+            q.val = m.val;
+        }
+        return q;
+    }
+
+    // The whole solve in one resident launch (cm_resident.hpp), in apply mode
+    // E on systems that were tuned (or come from a one-shot call), which leave
+    // the summation order to the engine.  Per pass it took, against the
+    // captured launches, 19 / 45 us at 100^2, 26 / 54 us at 45^3, 42 / 73 us
+    // at 64^3 and 86 / 115 us at 79^3 rows (FP64; FP32 50 / 91 us at 79^3),
+    // up to RS_MAX_ROWS, the most rows whose state the registers hold.  With a
+    // matrix in CSR the gathers go past the L2s entry by entry: 26 / 55 us at
+    // 100^2 but 72 / 73 us at 64^3, so beyond 65536 rows every matrix has to
+    // be in diagonals.  ran = false: not taken, or the grid could not be
+    // resident; x is untouched and the caller enqueues passes.  Launches being
+    // bracketed by profiling events are the passes', so a profiled solve does
+    // not come here.
+    int run_resident(double tol, int NMAX, int info_in, int trace_cap, bool zero_start, SolveState &fin, bool &ran)
+    {
+        ran = false;
+        if (!resident || prof.on || (variant == 2 && mode != 'E') || n > RS_MAX_ROWS) return CM_OK;
+        int dev = 0, cus = 0;
+        CM_HIP(hipGetDevice(&dev));
+        CM_HIP(hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev));
+        const int bsz = n <= RS_WGS * 256 ? 256 : 512;
+        const int rows = n <= RS_WGS * 512 ? 1 : n <= RS_WGS * 1024 ? 2 : 4;
+        const int grid = (n + bsz * rows - 1) / (bsz * rows);
+        if (grid > std::min(cus, RS_WGS)) return CM_OK;
+        if (!rs_slots) CM_TRY(dev_alloc(&rs_slots, (size_t)RS_SETS * RS_K * RS_WGS));
+        if (!rs_ctl) CM_TRY(dev_alloc(&rs_ctl, 1));
+        if (!rs_args) CM_TRY(dev_alloc(&rs_args, 1));
+        SolveState *out = &hst[1];
+        std::memset(out, 0, sizeof *out);
+        RsArgs<T, VA, VF> a;
+        std::memset(&a, 0, sizeof a);
+        a.n = n;
+        a.nmax = NMAX;
+        a.variant = variant;
+        a.maxmsteps = max_div_steps(variant, n);
+        a.info_in = info_in;
+        a.zero_start = zero_start ? 1 : 0;
+        a.trace_cap = trace_cap;
+        a.tol = tol;
+        a.eps = eps;
+        a.A = rs_mat(A, bsz, bsz * rows);
+        a.H = rs_mat(sym ? GT : H, bsz, bsz * rows);
+        a.G = rs_mat(G, bsz, bsz * rows);
+        if (n > RS_WGS * 256 && !(a.A.nd && a.H.nd && a.G.nd)) return CM_OK;
+        a.idv = idv;
+        a.b = b;
+        a.x = x;
+        T *ex[6] = {p, tm, pc, s, t1, sc};
+        for (int q = 0; q < 6; q++) a.ex[q] = ex[q];
+        CM_TRY(ensure_trace(trace_cap));
+        a.trace = trace_cap > 0 ? trace : nullptr;
+        a.slots = rs_slots;
+        a.ctl = rs_ctl;
+        a.out = out;
+        k_rs_prep<T, VA, VF><<<vec_grid(n), BS, 0, stream>>>(a, rs_args);
+        if (bsz == 256) k_rs_solve<T, VA, VF, 256, 1><<<grid, 256, 0, stream>>>(rs_args);
+        else if (rows == 1) k_rs_solve<T, VA, VF, 512, 1><<<grid, 512, 0, stream>>>(rs_args);
+        else if (rows == 2) k_rs_solve<T, VA, VF, 512, 2><<<grid, 512, 0, stream>>>(rs_args);
+        else k_rs_solve<T, VA, VF, 512, 4><<<grid, 512, 0, stream>>>(rs_args);
+        CM_HIP(hipGetLastError());
+        CM_HIP(hipStreamSynchronize(stream));
+        fin = *out;
+        ran = fin.done != 0;
+        return CM_OK;
+    }
+
+    // Writes the initial state (done = 0) of a solve of NMAX passes.
+    int begin(double tol, int NMAX, int info_in, int trace_cap)
+    {
+        CM_TRY(ensure_trace(trace_cap));
         SolveState init;
         std::memset(&init, 0, sizeof init);
         init.tol = tol;
@@ -1823,6 +1931,7 @@ static int tune_formats(KI &ki, int reps, hipEvent_t e0, hipEvent_t e1)
         CM_TRY(one(ki.U));
     }
     ki.drop_graphs();
+    ki.resident = true;
     return CM_OK;
 }
 
@@ -2784,10 +2893,15 @@ static int solve64(System &S, double tol, int NMAX, double *resval, int *iter, i
                    int trace_cap, int *ntrace)
 {
     K64 &k = *S.k64;
-    CM_TRY(k.begin(tol, NMAX, info ? *info : 0, trace ? trace_cap : 0));
-    k.setup_from_x();
+    const int info_in = info ? *info : 0, tcap = trace ? trace_cap : 0;
     SolveState fin;
-    CM_TRY(k.run(NMAX, fin));
+    bool ran;
+    CM_TRY(k.run_resident(tol, NMAX, info_in, tcap, false, fin, ran));
+    if (!ran) {
+        CM_TRY(k.begin(tol, NMAX, info_in, tcap));
+        k.setup_from_x();
+        CM_TRY(k.run(NMAX, fin));
+    }
     *iter = fin.iter;
     if (info) *info = fin.info;
     *resval = fin.rc / fin.ro;
@@ -2844,10 +2958,14 @@ static int solve_mixed(System &S, KI &ki, double tol, double inner_tol, int NMAX
         prev = rn;
         const double itol = stalled ? inner_tol : adaptive_inner_tol(inner_tol, tol, res0, rn);
         loose = itol > inner_tol;
-        CM_TRY(ki.begin(itol, NMAX, 0, 0));
-        ki.setup_zero();
         SolveState fin;
-        CM_TRY(ki.run(NMAX, fin));
+        bool ran;
+        CM_TRY(ki.run_resident(itol, NMAX, 0, 0, true, fin, ran));
+        if (!ran) {
+            CM_TRY(ki.begin(itol, NMAX, 0, 0));
+            ki.setup_zero();
+            CM_TRY(ki.run(NMAX, fin));
+        }
         out.inner_total += fin.ntrace;
         k_x_accum<<<g, BS, 0, S.stream>>>(n, k.x, ki.x);
         CM_HIP(hipGetLastError());
@@ -3873,6 +3991,7 @@ static int oneshot_formats(System &S)
         CM_TRY(set_format(*m, m->dia->nd >= DIA2_MIN_ND ? FMT_DIA2 : FMT_DIA, k.stream));
         CM_TRY(k.ensure_partials((m->n + BS - 1) / BS));
     }
+    k.resident = true;
     return CM_OK;
 }
 
