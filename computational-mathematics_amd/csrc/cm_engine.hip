@@ -2992,7 +2992,29 @@ using namespace cm;
 
 // ------------------------------------------------- persistent batched solves
 
-// Host side of k_batch_solve: device copies of the system descriptors and
+static BatchSys batch_sys(const K64 &k)
+{
+    const DevCsr<double> &H = k.sym ? k.GT : k.H;
+    return BatchSys{k.n, k.variant, max_div_steps(k.variant, k.n), 0, {H.ptr, k.G.ptr, k.A.ptr},
+                    {H.col, k.G.col, k.A.col}, {H.val, k.G.val, k.A.val}, k.idv};
+}
+
+// The two kernels over items sorted by size, largest first: the first nl are
+// beyond k_batch_small's LDS.  head: two ints.
+static int launch_batch(int nitems, int nl, int grid, const BatchSys *dsys, BatchItem *ditems, double *arena,
+                        size_t stride, int *head, int restart_true, hipStream_t s)
+{
+    k_zero_int<<<1, 2, 0, s>>>(head);
+    if (nl > 0)
+        k_batch_solve<<<std::min(grid, nl), PBS, 0, s>>>(nl, dsys, ditems, arena, stride, head, restart_true);
+    const int ns = nitems - nl;
+    if (ns > 0)
+        k_batch_small<<<std::min(grid, ns), BT_BS, 0, s>>>(ns, dsys, ditems + nl, arena, stride, head + 1, restart_true);
+    CM_HIP(hipGetLastError());
+    return CM_OK;
+}
+
+// Host side of the batch kernels: device copies of the system descriptors and
 // items, the per-workgroup arena and the items' b / x, grown on demand and
 // kept between calls.
 struct BatchRunner {
@@ -3002,8 +3024,12 @@ struct BatchRunner {
     double *arena = nullptr, *vec = nullptr;
     size_t arena_cap = 0, vec_cap = 0;  // doubles
     int *head = nullptr;
+    double *hvec = nullptr;  // pinned, at most STAGE_MAX bytes
+    size_t hvec_cap = 0;
+    static constexpr size_t STAGE_MAX = (size_t)64 << 20;
     ~BatchRunner()
     {
+        if (hvec) (void)hipHostFree(hvec);
         (void)hipFree(dsys);
         (void)hipFree(ditems);
         if (hitems) (void)hipHostFree(hitems);
@@ -3040,9 +3066,7 @@ struct BatchRunner {
         for (int q = 0; q < ns; q++) {
             const K64 &k = *systems[q]->k64;
             if (k.variant == 2 && k.mode != 'E') return fail(CM_ERR_UNSUPPORTED, "batched solves use apply mode E");
-            const DevCsr<double> &H = k.sym ? k.GT : k.H;
-            hs[q] = BatchSys{k.n, k.variant, max_div_steps(k.variant, k.n), 0, k.A.ptr, k.A.col, k.A.val,
-                             k.G.ptr, k.G.col, k.G.val, H.ptr, H.col, H.val, k.idv};
+            hs[q] = batch_sys(k);
             maxn = std::max(maxn, k.n);
         }
         // largest systems first (longest solves start early)
@@ -3050,12 +3074,14 @@ struct BatchRunner {
         for (int i = 0; i < nitems; i++) order[i] = i;
         std::stable_sort(order.begin(), order.end(),
                          [&](int a, int b) { return systems[sys_of[a]]->n > systems[sys_of[b]]->n; });
+        // vec: all right-hand sides, then all solutions, each in item order
         std::vector<size_t> off(nitems);
-        size_t tot = 0;
+        size_t half = 0;
         for (int i = 0; i < nitems; i++) {
-            off[i] = tot;
-            tot += 2 * (size_t)systems[sys_of[i]]->n;
+            off[i] = half;
+            half += (size_t)systems[sys_of[i]]->n;
         }
+        const size_t tot = 2 * half;
         int dev = 0, cus = 256;
         CM_HIP(hipGetDevice(&dev));
         CM_HIP(hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev));
@@ -3071,29 +3097,48 @@ struct BatchRunner {
         }
         CM_TRY(grow(&arena, arena_cap, stride * grid));
         CM_TRY(grow(&vec, vec_cap, tot));
-        if (!head) CM_HIP(hipMalloc((void **)&head, sizeof(int)));
+        if (!head) CM_HIP(hipMalloc((void **)&head, 2 * sizeof(int)));
+        // the vectors cross in one copy each way through pinned memory where
+        // they fit STAGE_MAX bytes of it: a copy per vector costs 5-8 us, 4 ms
+        // of a call with 192 items of some 10^3 rows
+        const bool staged = tot * sizeof(double) <= STAGE_MAX;
+        if (staged && tot > hvec_cap) {
+            if (hvec) (void)hipHostFree(hvec);
+            hvec = nullptr;
+            hvec_cap = 0;
+            CM_HIP(hipHostMalloc((void **)&hvec, tot * sizeof(double), hipHostMallocDefault));
+            hvec_cap = tot;
+        }
         for (int q = 0; q < nitems; q++) {
             const int i = order[q];
-            const int n = systems[sys_of[i]]->n;
-            double *db = vec + off[i], *dx = db + n;
-            CM_HIP(hipMemcpyAsync(db, B[i], (size_t)n * sizeof(double), hipMemcpyHostToDevice, s));
-            CM_HIP(hipMemcpyAsync(dx, X[i], (size_t)n * sizeof(double), hipMemcpyHostToDevice, s));
+            const size_t bytes = (size_t)systems[sys_of[i]]->n * sizeof(double);
+            double *db = vec + off[i], *dx = db + half;
+            if (staged) {
+                std::memcpy(hvec + off[i], B[i], bytes);
+                std::memcpy(hvec + half + off[i], X[i], bytes);
+            } else {
+                CM_HIP(hipMemcpyAsync(db, B[i], bytes, hipMemcpyHostToDevice, s));
+                CM_HIP(hipMemcpyAsync(dx, X[i], bytes, hipMemcpyHostToDevice, s));
+            }
             hitems[q] = BatchItem{sys_of[i], nmax[i], tol[i], db, dx, 0.0, 0, 0, 0, 0};
         }
+        if (staged) CM_HIP(hipMemcpyAsync(vec, hvec, tot * sizeof(double), hipMemcpyHostToDevice, s));
         CM_HIP(hipMemcpyAsync(dsys, hs.data(), ns * sizeof(BatchSys), hipMemcpyHostToDevice, s));
         CM_HIP(hipMemcpyAsync(ditems, hitems, (size_t)nitems * sizeof(BatchItem), hipMemcpyHostToDevice, s));
-        k_zero_int<<<1, 1, 0, s>>>(head);
-        k_batch_solve<<<grid, PBS, 0, s>>>(nitems, dsys, ditems, arena, stride, head, restart_true);
-        CM_HIP(hipGetLastError());
+        int nl = 0;  // items too large for k_batch_small come first
+        while (nl < nitems && systems[sys_of[order[nl]]]->n > BT_ROWS) nl++;
+        CM_TRY(launch_batch(nitems, nl, grid, dsys, ditems, arena, stride, head, restart_true, s));
         CM_HIP(hipMemcpyAsync(hitems, ditems, (size_t)nitems * sizeof(BatchItem), hipMemcpyDeviceToHost, s));
-        for (int q = 0; q < nitems; q++) {
-            const int i = order[q];
-            const int n = systems[sys_of[i]]->n;
-            CM_HIP(hipMemcpyAsync(X[i], vec + off[i] + n, (size_t)n * sizeof(double), hipMemcpyDeviceToHost, s));
-        }
+        if (staged) CM_HIP(hipMemcpyAsync(hvec + half, vec + half, half * sizeof(double), hipMemcpyDeviceToHost, s));
+        else
+            for (int i = 0; i < nitems; i++)
+                CM_HIP(hipMemcpyAsync(X[i], vec + half + off[i], (size_t)systems[sys_of[i]]->n * sizeof(double),
+                                      hipMemcpyDeviceToHost, s));
         CM_HIP(hipStreamSynchronize(s));
         for (int q = 0; q < nitems; q++) {
             const int i = order[q];
+            if (staged)
+                std::memcpy(X[i], hvec + half + off[i], (size_t)systems[sys_of[i]]->n * sizeof(double));
             if (resval) resval[i] = hitems[q].resval;
             if (iter) iter[i] = hitems[q].iter;
             if (info && hitems[q].info >= 0) info[i] = hitems[q].info;  // untouched when NMAX < 0
@@ -3571,9 +3616,7 @@ int cm_batch_solve_noalloc(int nitems, const cm_system *systems, const double *c
                                             " distinct systems");
             const K64 &k = *p->k64;
             if (k.variant == 2 && k.mode != 'E') return fail(CM_ERR_UNSUPPORTED, "batched solves use apply mode E");
-            const DevCsr<double> &H = k.sym ? k.GT : k.H;
-            g_na_sys[ns] = BatchSys{k.n, k.variant, max_div_steps(k.variant, k.n), 0, k.A.ptr, k.A.col, k.A.val,
-                                    k.G.ptr, k.G.col, k.G.val, H.ptr, H.col, H.val, k.idv};
+            g_na_sys[ns] = batch_sys(k);
             g_na_sysptr[ns++] = p;
             maxn = std::max(maxn, k.n);
         }
@@ -3603,9 +3646,9 @@ int cm_batch_solve_noalloc(int nitems, const cm_system *systems, const double *c
     double *arena = reinterpret_cast<double *>(base + NA_ARENA);
     CM_HIP(hipMemcpyAsync(dsys, g_na_sys, ns * sizeof(BatchSys), hipMemcpyHostToDevice, s));
     CM_HIP(hipMemcpyAsync(ditems, g_na_items, (size_t)nitems * sizeof(BatchItem), hipMemcpyHostToDevice, s));
-    k_zero_int<<<1, 1, 0, s>>>(head);
-    k_batch_solve<<<grid, PBS, 0, s>>>(nitems, dsys, ditems, arena, stride, head, restart_true);
-    CM_HIP(hipGetLastError());
+    int nl = 0;  // items too large for k_batch_small come first
+    while (nl < nitems && g_na_sysptr[g_na_items[nl].sys]->n > BT_ROWS) nl++;
+    CM_TRY(launch_batch(nitems, nl, grid, dsys, ditems, arena, stride, head, restart_true, s));
     CM_HIP(hipMemcpyAsync(g_na_items, ditems, (size_t)nitems * sizeof(BatchItem), hipMemcpyDeviceToHost, s));
     CM_HIP(hipStreamSynchronize(s));
     for (int q = 0; q < nitems; q++) {

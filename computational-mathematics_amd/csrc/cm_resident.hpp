@@ -111,6 +111,14 @@ __device__ __forceinline__ double rs_uni(double v)
     return v;
 }
 
+// A pointer read from a table, known to point to device memory: its loads are
+// global ones, not flat ones (which also wait for LDS).
+template <class X>
+__device__ __forceinline__ X *rs_glob(X *p)
+{
+    return (X *)(__attribute__((address_space(1))) X *)p;
+}
+
 // Control words of one launch, cleared by k_rs_prep.
 struct RsCtl {
     unsigned join;  // arrivals; top bit: closed
@@ -256,8 +264,8 @@ __device__ __forceinline__ void rs_tile(RsConst<RsMat<V>> m, int c0, int re, int
         j[q] = -1;
         ev[q] = 0;
         if (k < re) {
-            j[q] = m->col[k];
-            ev[q] = load_val<V, Acc>(m->val, k);
+            j[q] = rs_glob(m->col)[k];
+            ev[q] = load_val<V, Acc>(rs_glob(m->val), k);
         }
     }
 }
@@ -273,8 +281,8 @@ __device__ __forceinline__ void rs_ahead(RsConst<RsMat<V>> m, int rs, int re, in
 #pragma unroll
         for (int q = 0; q < R; q++) {
             const int i = row0 + q * BSZ + (int)threadIdx.x;
-            f.a[q] = m->ptr[min(i, n)];
-            f.e[q] = m->ptr[min(i + 1, n)];
+            f.a[q] = rs_glob(m->ptr)[min(i, n)];
+            f.e[q] = rs_glob(m->ptr)[min(i + 1, n)];
         }
     }
 }
@@ -288,7 +296,7 @@ __device__ __forceinline__ void rs_hold(RsConst<RsMat<V>> m, int n, int row0, V 
         const int i = row0 + q * BSZ + (int)threadIdx.x;
 #pragma unroll
         for (int d = 0; d < ND; d++)
-            dv[q][d] = d < m->nd && i < n ? *rs_at(m->dval, (unsigned)(d * m->ldn + i)) : (V)0.0f;
+            dv[q][d] = d < m->nd && i < n ? *rs_at(rs_glob(m->dval), (unsigned)(d * m->ldn + i)) : (V)0.0f;
     }
 }
 
@@ -347,7 +355,7 @@ __device__ __forceinline__ void rs_rows(RsConst<RsMat<V>> m, const V (&dv)[R][ND
         for (int d = 0; d < RS_DC; d++)
 #pragma unroll
             for (int q = 0; q < R; q++)
-                v[q][d] = *rs_at(m->dval, (unsigned)(min(d0 + d, nd - 1) * m->ldn + min(row0 + q * BSZ + tid, n - 1)));
+                v[q][d] = *rs_at(rs_glob(m->dval), (unsigned)(min(d0 + d, nd - 1) * m->ldn + min(row0 + q * BSZ + tid, n - 1)));
 #pragma unroll
         for (int d = 0; d < RS_DC; d++)
             if (d0 + d < nd) {
@@ -385,7 +393,7 @@ __device__ __forceinline__ void rs_rows(RsConst<RsMat<V>> m, const V (&dv)[R][ND
 #pragma unroll
     for (int q = 0; q < R; q++) {
         const int i = row0 + q * BSZ + tid;
-        if (m->rowscale && i < n) y[q] *= (Acc)m->rowscale[i];
+        if (m->rowscale && i < n) y[q] *= (Acc)rs_glob(m->rowscale)[i];
         if (i >= n) y[q] = 0;  // rows past n took other rows' values
     }
 }
@@ -531,9 +539,9 @@ __global__ __launch_bounds__(BSZ) void k_rs_solve(const RsArgs<T, VA, VF> *args)
         const int i = row0 + q * BSZ + tid;
         x[q] = r[q] = dv[q] = r0[q] = p[q] = v[q] = w[q] = (T)0;
         if (i < n) {
-            dv[q] = g->idv[i];
-            r[q] = g->b[i];
-            if (!g->zero_start) x[q] = g->x[i];
+            dv[q] = rs_glob(g->idv)[i];
+            r[q] = rs_glob(g->b)[i];
+            if (!g->zero_start) x[q] = rs_glob(g->x)[i];
         }
     }
     // diagonals held in registers: a 7-point matrix's and its PDFIIM factors'
@@ -561,10 +569,10 @@ __global__ __launch_bounds__(BSZ) void k_rs_solve(const RsArgs<T, VA, VF> *args)
         // steps they would take the registers that hold the values
         asm volatile("" : "+s"(g));
         Acc y[R];
-        const T *src = g->x;
+        const T *src = rs_glob(g->x);
         if (step != 6) {
-            T *const ex[3] = {step == 2 ? g->ex[0] : g->ex[3], step == 2 ? g->ex[1] : g->ex[4],
-                              step == 2 ? g->ex[2] : g->ex[5]};
+            T *const ex[3] = {rs_glob(step == 2 ? g->ex[0] : g->ex[3]), rs_glob(step == 2 ? g->ex[1] : g->ex[4]),
+                              rs_glob(step == 2 ? g->ex[2] : g->ex[5])};
             rs_rows<T, VF, Acc, BSZ, R, 17>(&g->H, dh, tile, lo[0], hi[0], n, row0, ex[0], win, prod, dead, y);
             rs_ahead<VF, Acc, BSZ, R>(&g->G, lo[1], hi[1], n, row0, tile);
 #pragma unroll
@@ -621,7 +629,7 @@ __global__ __launch_bounds__(BSZ) void k_rs_solve(const RsArgs<T, VA, VF> *args)
                 sm[0] += (double)r[q] * (double)r[q];
             }
         }
-        rs_allsum<BSZ>(sm, g->slots, set, red[set], dead);
+        rs_allsum<BSZ>(sm, rs_glob(g->slots), set, red[set], dead);
         if (rs_uni(*dead)) return;
         if (step == 2) {
             alpha = m1 / sm[0];
@@ -641,13 +649,13 @@ __global__ __launch_bounds__(BSZ) void k_rs_solve(const RsArgs<T, VA, VF> *args)
                 x[q] = x[q] + al * w[q];
                 r[q] = r[q] + na * v[q];  // s
                 if (i < n) {
-                    rs_put(g->ex[3] + i, r[q]);
+                    rs_put(rs_glob(g->ex[3]) + i, r[q]);
 #pragma unroll
-                    for (int e = 0; e < 3; e++) rs_put_bits(g->ex[e] + i, RsBits<T>::MARK);
+                    for (int e = 0; e < 3; e++) rs_put_bits(rs_glob(g->ex[e]) + i, RsBits<T>::MARK);
                 }
             }
             if (tid < RS_K)
-                rs_put_bits(g->slots + ((size_t)(3 + (par ^ 1)) * RS_K + tid) * RS_WGS + blockIdx.x,
+                rs_put_bits(rs_glob(g->slots) + ((size_t)(3 + (par ^ 1)) * RS_K + tid) * RS_WGS + blockIdx.x,
                             RsBits<double>::MARK);
             step = 5;
             continue;
@@ -708,15 +716,15 @@ __global__ __launch_bounds__(BSZ) void k_rs_solve(const RsArgs<T, VA, VF> *args)
         for (int q = 0; q < R; q++) {
             const int i = row0 + q * BSZ + tid;
             if (i < n) {
-                rs_put(g->ex[0] + i, p[q]);
+                rs_put(rs_glob(g->ex[0]) + i, p[q]);
                 if (step == 5)
 #pragma unroll
-                    for (int e = 3; e < 6; e++) rs_put_bits(g->ex[e] + i, RsBits<T>::MARK);
+                    for (int e = 3; e < 6; e++) rs_put_bits(rs_glob(g->ex[e]) + i, RsBits<T>::MARK);
             }
         }
         if (step == 5) {
             if (tid < RS_K)
-                rs_put_bits(g->slots + ((size_t)(1 + par) * RS_K + tid) * RS_WGS + blockIdx.x, RsBits<double>::MARK);
+                rs_put_bits(rs_glob(g->slots) + ((size_t)(1 + par) * RS_K + tid) * RS_WGS + blockIdx.x, RsBits<double>::MARK);
             par ^= 1;
         }
         step = 2;
@@ -724,7 +732,7 @@ __global__ __launch_bounds__(BSZ) void k_rs_solve(const RsArgs<T, VA, VF> *args)
 #pragma unroll
     for (int q = 0; q < R; q++) {
         const int i = row0 + q * BSZ + tid;
-        if (i < n && (g->nmax > 0 || g->zero_start)) g->x[i] = x[q];
+        if (i < n && (g->nmax > 0 || g->zero_start)) rs_glob(g->x)[i] = x[q];
     }
     if (blockIdx.x == 0 && tid == 0) {
         SolveState *o = g->out;
