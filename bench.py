@@ -821,7 +821,7 @@ def bench_single(args, w):
     # timed region: only the dominant kernel's launches carry events, and only in the first
     # SAMPLE_PASSES passes of each solve (launched kernel by kernel); the other passes replay from
     # the captured graphs, as in an unprofiled solve.  A dominant category of many launches per pass
-    # (the level-scheduled triangular solves: thousands per pass) is timed in separate solves
+    # (thousands of small ones, say) is timed in separate solves
     # instead: events around each of its launches would slow the timed solves themselves.
     profiled_passes = max(1, stats["A"][0] // 2)  # passes of the two profiled solves (two A products each)
     kernel_timing = args.kernel_timing
@@ -897,9 +897,9 @@ def bench_single(args, w):
     d_gbs = by / ms / 1e6
     kname = CAT_KERNELS.get(dom, dom)
     mode = w.get("mode", "E")
-    if dom == "LU":  # mode C's L / U products, or modes I / J's level-scheduled triangular solves
+    if dom == "LU":  # mode C's L / U products, or modes I / J's triangular solves
         if mode in ("I", "J"):
-            kname = "cm::k_trsv_level<double, double> (one launch per dependency level)"
+            kname = "cm::k_trsv_flow<double, double> (one launch per triangle)"
         else:
             fmt_l = formats.get(64, {}).get("L", "staged") if tuned else "staged"
             if fmt_l in ("dia", "dia2"):

@@ -109,15 +109,6 @@ __global__ __launch_bounds__(BS) void k_gather_vals(long long cnt, const int *__
     }
 }
 
-// z = a .* d (mode I of the ACIFIM apply)
-template <class T>
-__global__ __launch_bounds__(BS) void k_vmul(int n, const T *__restrict__ a, const T *__restrict__ d,
-                                             T *__restrict__ z, const SolveState *st)
-{
-    if (st && st->done) return;
-    for (int i = blockIdx.x * BS + threadIdx.x; i < n; i += gridDim.x * BS) z[i] = a[i] * d[i];
-}
-
 // Sets *bad to 1 when a stored column lies outside [0, n) (the upload's
 // column check, on the device).
 __global__ __launch_bounds__(BS) void k_col_range(long long nnz, const int *__restrict__ col, int n, int *bad)
@@ -383,13 +374,12 @@ struct DevCsr {
     bool use_dia = false;              // products through spmv_dia
     bool dia2 = false;                 // ... in its second variant (FMT_DIA2)
     bool block_dia = false;            // block products (SpMM) through spmm_dia
-    int nlev = 0;
+    int nlev = 0;  // dependency levels
     bool lower = false;  // the level schedule's triangle (lower: rows read smaller columns)
     int *lrows = nullptr;
-    std::vector<int> loff;
-    int *dloff = nullptr;         // loff on the device (read by the run-of-levels kernel)
-    std::vector<long long> lnnz;  // per level: the triangle's entries of its rows
-    int lpr = 1;                  // lanes per row of the level kernel
+    int nchunk = 0;
+    int4 *crow = nullptr;  // the triangular solve's chunks: nchunk x (WAVE / lpr) of {row, first entry, end, 0}
+    int lpr = 1;          // lanes per row of the triangular solve
     // the triangle's entries in level order (tptr indexed by level position;
     // tsrc: CSR positions; tval: this copy's values gathered through tsrc)
     int *tptr = nullptr, *tcol = nullptr, *tsrc = nullptr;
@@ -409,7 +399,7 @@ struct DevCsr {
             if (slots) b += slots->bytes();
             if (dia) b += dia->bytes();
             b += (size_t)(n + 1 + 2 * (nblk + 1)) * sizeof(int) + (size_t)nnz * sizeof(int) + (lrows ? (size_t)n * sizeof(int) : 0);
-            if (dloff) b += (size_t)(nlev + 1) * sizeof(int);
+            if (crow) b += (size_t)nchunk * (WAVE / lpr) * sizeof(int4);
             if (d16) b += (size_t)(nnz + 2 * CSR_PAD) * sizeof(uint16_t) + (size_t)nblk * sizeof(int);
         }
         return b;
@@ -421,7 +411,7 @@ struct DevCsr {
             (void)hipFree(col);
             (void)hipFree(blk);
             (void)hipFree(lrows);
-            (void)hipFree(dloff);
+            (void)hipFree(crow);
             (void)hipFree(d16);
             (void)hipFree(cbase);
             (void)hipFree(tptr);
@@ -435,7 +425,8 @@ struct DevCsr {
         (void)hipFree(dval);
         (void)hipFree(rval);
         (void)hipFree(lval);
-        ptr = col = blk = lrows = cbase = dloff = nullptr;
+        ptr = col = blk = lrows = cbase = nullptr;
+        crow = nullptr;
         tptr = tcol = tsrc = nullptr;
         ntri = 0;
         d16 = nullptr;
@@ -517,9 +508,8 @@ static int cast_csr(DevCsr<V> &dst, const DevCsr<double> &src, hipStream_t s)
     dst.nlev = src.nlev;
     dst.lower = src.lower;
     dst.lrows = src.lrows;
-    dst.loff = src.loff;
-    dst.dloff = src.dloff;
-    dst.lnnz = src.lnnz;
+    dst.crow = src.crow;
+    dst.nchunk = src.nchunk;
     dst.lpr = src.lpr;
     dst.tptr = src.tptr;
     dst.tcol = src.tcol;
@@ -938,9 +928,7 @@ static int build_levels(DevCsr<double> &m, const int *ptr, const int *col, bool 
     LevelSchedule L = level_schedule(m.n, ptr, col, lower, false);
     m.nlev = L.nlev;
     m.lower = lower;
-    m.loff = L.loff;
     CM_TRY(dev_upload(&m.lrows, L.rows.data(), (size_t)m.n, s));
-    CM_TRY(dev_upload(&m.dloff, L.loff.data(), L.loff.size(), s));
     // the triangle's entries in level order
     const int n = m.n;
     DevTemps tmp;
@@ -959,17 +947,21 @@ static int build_levels(DevCsr<double> &m, const int *ptr, const int *col, bool 
     CM_HIP(hipMemcpyAsync(tp.data(), m.tptr, tp.size() * sizeof(int), hipMemcpyDeviceToHost, s));
     CM_HIP(hipStreamSynchronize(s));
     m.ntri = tp[n];
-    m.lnnz.assign(L.nlev, 0);  // the triangle's entries each level's rows hold (read by its launch)
-    for (int l = 0; l < L.nlev; l++) m.lnnz[l] = tp[L.loff[l + 1]] - tp[L.loff[l]];
     CM_TRY(dev_alloc(&m.tcol, (size_t)m.ntri));
     CM_TRY(dev_alloc(&m.tsrc, (size_t)m.ntri));
     CM_TRY(dev_alloc(&m.tval, (size_t)m.ntri));
     k_tri_fill<<<g, BS, 0, s>>>(n, m.lrows, m.ptr, m.col, lower, m.tptr, m.tcol, m.tsrc);
     if (m.ntri) k_gather_vals<double><<<long_grid(m.ntri), BS, 0, s>>>(m.ntri, m.tsrc, m.val, m.tval);
-    // lanes per row: the power of two at or above the triangle's mean row length, 1..16
-    const double mean = m.n ? (double)m.ntri / m.n : 0.0;
-    m.lpr = 1;
-    while (m.lpr < 16 && m.lpr < mean) m.lpr *= 2;
+    m.lpr = trsv_lanes((double)m.ntri / m.n);
+    // chunks of one wave's rows, none across two levels (padded with row -1)
+    const int rpw = WAVE / m.lpr;
+    std::vector<int4> crow;
+    for (int l = 0; l < L.nlev; l++) {
+        for (int q = L.loff[l]; q < L.loff[l + 1]; q++) crow.push_back(make_int4(L.rows[q], tp[q], tp[q + 1], 0));
+        while (crow.size() % rpw) crow.push_back(make_int4(-1, 0, 0, 0));
+    }
+    m.nchunk = (int)(crow.size() / rpw);
+    CM_TRY(dev_upload(&m.crow, crow.data(), crow.size(), s));
     CM_HIP(hipGetLastError());
     CM_HIP(hipStreamSynchronize(s));  // before the temporaries are freed
     return CM_OK;
@@ -982,6 +974,15 @@ static int max_div_steps(int variant, int n)
     if (variant == 2) return std::min(std::max(n, 2000) / 50, 40);
     return std::min(std::max(n, 500) / 50, 20);
 }
+
+// A triangular solve launches this many times the workgroups it wants at
+// work, which are those of one XCD (workgroups go round the XCDs in turn).
+// More waves than a few levels' chunks only look for rows far ahead, and
+// their looks slow the others': an apply (L and U) of 64^3 rows took 1208,
+// 861, 779, 762, 944 and 1431 us with 1, 2, 3, 5, 8 and 15 levels' chunks at
+// work, of 128^3 rows 3241, 2639, 2746, 5259 and 12435 us with 1, 2, 3, 5 and 8
+// (2106 and 5788 us with a launch per level).
+constexpr int TRSV_XCDS = 8;
 
 // Passes per captured hipGraph (besides the one-pass graph).
 constexpr int GRAPH_PASSES = 4;
@@ -1105,6 +1106,7 @@ struct Krylov {
     // when no launch is being bracketed by profiling events
     bool use_graph = true;
     hipGraphExec_t g1 = nullptr, gN = nullptr;
+    TrsvCtl *trsv_ctl = nullptr;  // control words of an apply's two triangular solves (modes I, J)
     bool resident = false;       // whole solves in one launch (tuned systems; run_resident)
     double *rs_slots = nullptr;  // reduction slots and control words of the resident solve (first use)
     RsCtl *rs_ctl = nullptr;
@@ -1125,6 +1127,7 @@ struct Krylov {
         for (T *q : bufs) (void)hipFree(q);
         (void)hipFree(partials);
         (void)hipFree(trace);
+        (void)hipFree(trsv_ctl);
         (void)hipFree(rs_slots);
         (void)hipFree(rs_ctl);
         (void)hipFree(rs_args);
@@ -1159,6 +1162,7 @@ struct Krylov {
         const int maxblk = std::max(nblk_a, MAX_RED_BLOCKS);
         CM_HIP(hipMalloc((void **)&partials, (size_t)maxblk * 4 * sizeof(double)));
         partials_cap = (size_t)maxblk * 4;
+        if (variant == 2 && (mode == 'I' || mode == 'J')) CM_TRY(dev_alloc(&trsv_ctl, 2));
         for (auto &e : ev) CM_HIP(hipEventCreateWithFlags(&e, hipEventDisableTiming));
         return CM_OK;
     }
@@ -1328,15 +1332,24 @@ struct Krylov {
                   [&] { k_finalize<Epi::K, Epi><<<1, FBS, 0, stream>>>(m.nblk, partials, kst, epi); });
     }
 
-    // x = T^{-1} b for a unit triangular factor with its level schedule: one
-    // launch per level, or one workgroup for a run of at least two consecutive
-    // levels that each take at most TRSV_RUN_STEPS steps of its lane groups
-    void trsv(const DevCsr<VF> &m, const T *bin, T *xout, bool use_state)
+    // x = T^{-1} (b .* dscale) for a triangular factor in level order (dscale
+    // null: T^{-1} b); the q-th of the pair that trsv_prep readied
+    void trsv(const DevCsr<VF> &m, const T *bin, const T *dscale, T *xout, int q, bool use_state)
     {
-        const SolveState *gate = use_state ? st : nullptr;
-        const int run_rows = TRSV_RUN_STEPS * (TRSV_RUN_THREADS / m.lpr);
-        auto small = [&](int l) { return m.loff[l + 1] - m.loff[l] <= run_rows; };
-        auto lanes = [&](auto go) {
+        // the triangle's entries (value + column), row list and row pointers once, and per row
+        // the right-hand side read, the solution written and read back
+        const double by = (double)m.ntri * (sizeof(VF) + 4.0) +
+                          (double)n * (4.0 + 8.0 + (dscale ? 4.0 : 3.0) * sizeof(T));
+        timed(KC_LU, by, [&] {
+            auto go = [&](auto lz) {
+                constexpr int LPR = decltype(lz)::value;
+                // waves for two and a half levels' chunks
+                const long long waves = std::min<long long>(512, 5LL * m.nchunk / (2LL * std::max(1, m.nlev)) + 4);
+                const int g = (int)(TRSV_XCDS * ((waves + TRSV_BS / WAVE - 1) / (TRSV_BS / WAVE)));
+                k_trsv_flow<T, VF, LPR><<<g, TRSV_BS, 0, stream>>>(m.nchunk, m.crow, m.tcol, m.tval, m.rowscale,
+                                                                  bin, dscale, xout, trsv_ctl + q,
+                                                                  use_state ? st : nullptr, use_state ? st : nullptr);
+            };
             switch (m.lpr) {
             case 1: go(std::integral_constant<int, 1>{}); break;
             case 2: go(std::integral_constant<int, 2>{}); break;
@@ -1344,41 +1357,7 @@ struct Krylov {
             case 8: go(std::integral_constant<int, 8>{}); break;
             default: go(std::integral_constant<int, 16>{}); break;
             }
-        };
-        // the levels' entries (value + column), row list and row pointers, and per row the
-        // right-hand side read, the solution written and (once over all levels) read back
-        auto level_bytes = [&](int l) {
-            const int cnt = m.loff[l + 1] - m.loff[l];
-            return (double)m.lnnz[l] * (sizeof(VF) + 4.0) + (double)cnt * (4.0 + 8.0 + 3.0 * sizeof(T));
-        };
-        for (int l = 0; l < m.nlev;) {
-            int l2 = l;
-            while (l2 < m.nlev && small(l2)) l2++;
-            if (l2 - l >= 2 && m.dloff) {
-                double by = 0.0;
-                for (int q = l; q < l2; q++) by += level_bytes(q);
-                timed(KC_LU, by, [&] {
-                    lanes([&](auto lz) {
-                        constexpr int LPR = decltype(lz)::value;
-                        k_trsv_run<T, VF, LPR><<<1, TRSV_RUN_THREADS, 0, stream>>>(
-                            l, l2, m.dloff, m.lrows, m.tptr, m.tcol, m.tval, m.rowscale, bin, xout, gate);
-                    });
-                });
-                l = l2;
-                continue;
-            }
-            const int cnt = m.loff[l + 1] - m.loff[l];
-            const int q0 = m.loff[l];
-            timed(KC_LU, level_bytes(l), [&] {
-                lanes([&](auto lz) {
-                    constexpr int LPR = decltype(lz)::value;
-                    const int g = (int)(((long long)cnt * LPR + BS - 1) / BS);
-                    k_trsv_level<T, VF, LPR><<<g, BS, 0, stream>>>(cnt, m.lrows + q0, m.tptr + q0, m.tcol, m.tval,
-                                                                   m.rowscale, bin, xout, gate);
-                });
-            });
-            l++;
-        }
+        });
     }
 
     // out = M in, per the reference's apply (ACIFIM/src/bicgstab.cpp:372-428);
@@ -1392,17 +1371,12 @@ struct Krylov {
             return;
         }
         if (mode == 'I' || mode == 'J') {
-            // I: t1 = L^{-1} b; t2 = t1 .* IDv; x = U^{-1} t2.   J: x = U^{-1} L^{-1} b.
-            trsv(L, in, t1, use_state);
-            if (mode == 'I') {
-                const int g = vec_grid(n);
-                timed(KC_VEC, 3.0 * sizeof(T) * n, [&] {
-                    k_vmul<T><<<g, BS, 0, stream>>>(n, t1, idv, t2, use_state ? st : nullptr);
-                });
-                trsv(U, t2, out, use_state);
-            } else {
-                trsv(U, t1, out, use_state);
-            }
+            // I: t1 = L^{-1} b; x = U^{-1} (t1 .* IDv).   J: x = U^{-1} L^{-1} b.
+            timed(KC_VEC, 2.0 * sizeof(T) * n, [&] {
+                k_trsv_prep<T><<<vec_grid(n), BS, 0, stream>>>(n, t1, out, trsv_ctl, use_state ? st : nullptr);
+            });
+            trsv(L, in, nullptr, t1, 0, use_state);
+            trsv(U, t1, mode == 'I' ? idv : nullptr, out, 1, use_state);
             return;
         }
         // mode C: t1 = H b; repeat: t1 += H (b - L t1); t2 = t1 .* IDv;
@@ -1686,6 +1660,7 @@ struct Krylov {
         }
         CM_HIP(hipStreamSynchronize(stream));
         CM_HIP(hipGetLastError());
+        if (fin_state.stalled) return fail(CM_ERR_HIP, "a triangular solve gave up waiting for a row");
         if (prof.on) prof.collect(fin_state.ntrace);
         if (!fin_state.done) return fail(CM_ERR_HIP, "solve state did not reach done");
         return CM_OK;
@@ -3943,6 +3918,11 @@ int cm_system_apply(cm_system h, const double *v, double *out)
     CM_HIP(hipMemcpyAsync(out, k.sc, (size_t)S.n * sizeof(double), hipMemcpyDeviceToHost, S.stream));
     CM_HIP(hipStreamSynchronize(S.stream));
     CM_HIP(hipGetLastError());
+    if (k.trsv_ctl) {
+        TrsvCtl c[2];
+        CM_HIP(hipMemcpy(c, k.trsv_ctl, sizeof c, hipMemcpyDeviceToHost));
+        if (c[0].fail || c[1].fail) return fail(CM_ERR_HIP, "a triangular solve gave up waiting for a row");
+    }
     return CM_OK;
 }
 

@@ -47,6 +47,7 @@ struct SolveState {
     double res_outer;  // ||b - A x|| of the last refinement residual (mixed path)
     int iter, nmax, stag, msteps, maxmsteps, info, done, variant;
     int ntrace, trace_cap;
+    int stalled, pad;  // a triangular solve gave up waiting (never seen; an error)
     double *trace;  // device array of trace_cap doubles or null
 };
 
