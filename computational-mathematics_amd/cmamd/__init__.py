@@ -16,6 +16,7 @@ from __future__ import annotations
 
 import ctypes as C
 import os
+import weakref
 from dataclasses import dataclass
 
 import numpy as np
@@ -142,13 +143,12 @@ def _type_host(lib):
 
 
 def _take(lib, p, count, dtype):
-    """Copy a new[]-allocated array into numpy and release it."""
+    """A numpy array over a new[]-allocated one, released with its last view."""
     if not p:
         return None
-    ctype = C.c_double if dtype == np.float64 else C.c_int
-    arr = np.ctypeslib.as_array(C.cast(p, C.POINTER(ctype)), (max(count, 1),))[:count].copy()
-    (lib.cm_free_d if dtype == np.float64 else lib.cm_free_i)(p)
-    return arr
+    buf = ((C.c_double if dtype == np.float64 else C.c_int) * max(count, 1)).from_address(p)
+    weakref.finalize(buf, lib.cm_free_d if dtype == np.float64 else lib.cm_free_i, p)
+    return np.frombuffer(buf, dtype=dtype)[:count]
 
 
 def _take_csr(lib, n, pv, pj, pi):

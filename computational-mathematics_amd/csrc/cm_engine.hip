@@ -150,19 +150,11 @@ class Stager {
     int upload(void *dst, const void *src, size_t bytes, hipStream_t s)
     {
         std::lock_guard<std::mutex> lk(mu);
-        if (!buf[0]) {
-            for (auto &b : buf) CM_HIP(hipHostMalloc((void **)&b, CHUNK, hipHostMallocDefault));
-            for (int h = 0; h < STAGE_HELPERS; h++) std::thread([this] { help(); }).detach();
-        }
+        CM_TRY(start());
         for (size_t off = 0; off < bytes; next = (next + 1) % NBUF) {
             const int b = next;
             const size_t len = std::min(CHUNK, bytes - off);
-            if (ev[b]) {  // the chunk's previous copy must have left it
-                const hipError_t e = hipEventSynchronize(ev[b]);
-                (void)hipEventDestroy(ev[b]);
-                ev[b] = nullptr;
-                if (e != hipSuccess) return fail(CM_ERR_HIP, "staged upload wait failed");
-            }
+            CM_TRY(drain(b));  // the chunk's previous copy must have left it
             copy(buf[b], (const char *)src + off, len);
             CM_HIP(hipMemcpyAsync((char *)dst + off, buf[b], len, hipMemcpyHostToDevice, s));
             CM_HIP(hipEventCreateWithFlags(&ev[b], hipEventDisableTiming));  // on the stream's (current) device
@@ -172,8 +164,61 @@ class Stager {
         return CM_OK;
     }
 
+    // The other way: a chunk is copied out of its pinned buffer by the threads
+    // while the next one arrives.  The destination is fresh memory as a rule,
+    // whose first touch costs more than the copy: four threads share it.
+    // Returns with the data in place.
+    int download(void *dst, const void *src, size_t bytes, hipStream_t s)
+    {
+        std::lock_guard<std::mutex> lk(mu);
+        CM_TRY(start());
+        int b[2];
+        size_t off[2], len[2];
+        size_t asked = 0;
+        int head = 0, n = 0;
+        auto ask = [&]() -> int {
+            const int q = (head + n) % 2;
+            b[q] = next;
+            next = (next + 1) % NBUF;
+            CM_TRY(drain(b[q]));
+            off[q] = asked;
+            len[q] = std::min(CHUNK / 4, bytes - asked);
+            CM_HIP(hipMemcpyAsync(buf[b[q]], (const char *)src + asked, len[q], hipMemcpyDeviceToHost, s));
+            CM_HIP(hipEventCreateWithFlags(&ev[b[q]], hipEventDisableTiming));
+            CM_HIP(hipEventRecord(ev[b[q]], s));
+            asked += len[q];
+            n++;
+            return CM_OK;
+        };
+        CM_TRY(ask());
+        while (n) {
+            if (asked < bytes) CM_TRY(ask());
+            CM_TRY(drain(b[head]));
+            copy((char *)dst + off[head], buf[b[head]], len[head]);
+            head = 1 - head;
+            n--;
+        }
+        return CM_OK;
+    }
+
   private:
-    std::mutex mu;  // one upload at a time
+    int start()
+    {
+        if (buf[0]) return CM_OK;
+        for (auto &b : buf) CM_HIP(hipHostMalloc((void **)&b, CHUNK, hipHostMallocDefault));
+        for (int h = 0; h < STAGE_HELPERS; h++) std::thread([this] { help(); }).detach();
+        return CM_OK;
+    }
+    // the chunk's last copy is done
+    int drain(int b)
+    {
+        if (!ev[b]) return CM_OK;
+        const hipError_t e = hipEventSynchronize(ev[b]);
+        (void)hipEventDestroy(ev[b]);
+        ev[b] = nullptr;
+        return e == hipSuccess ? CM_OK : fail(CM_ERR_HIP, "staged copy wait failed");
+    }
+    std::mutex mu;  // one transfer at a time
     char *buf[NBUF] = {};
     hipEvent_t ev[NBUF] = {};  // recorded behind each chunk's last copy
     int next = 0;              // the chunk filled next
@@ -227,6 +272,17 @@ static int copy_h2d(T *d, const T *h, size_t count, hipStream_t s)
     const size_t bytes = count * sizeof(T);
     if (bytes >= Stager::MIN_BYTES) return Stager::get().upload(d, h, bytes, s);
     CM_HIP(hipMemcpyAsync(d, h, bytes, hipMemcpyHostToDevice, s));
+    return CM_OK;
+}
+
+// Device to host (pageable), large arrays through pinned chunks; small ones
+// are only enqueued.
+template <class T>
+static int copy_d2h(T *h, const T *d, size_t count, hipStream_t s)
+{
+    const size_t bytes = count * sizeof(T);
+    if (bytes >= Stager::MIN_BYTES) return Stager::get().download(h, d, bytes, s);
+    if (bytes) CM_HIP(hipMemcpyAsync(h, d, bytes, hipMemcpyDeviceToHost, s));
     return CM_OK;
 }
 
@@ -2518,7 +2574,7 @@ struct BlockSolver : BlockBase {
     {
         const int g = (int)std::min<size_t>(((size_t)n * KB + BS - 1) / BS, 8192);
         k_deinterleave<KB><<<g, BS, 0, stream>>>(n, ncols, b64.x, cm);
-        CM_HIP(hipMemcpyAsync(X, cm, (size_t)n * ncols * sizeof(double), hipMemcpyDeviceToHost, stream));
+        CM_TRY(copy_d2h(X, cm, (size_t)n * ncols, stream));
         CM_HIP(hipStreamSynchronize(stream));
         return CM_OK;
     }
@@ -3126,30 +3182,65 @@ struct BatchRunner {
 
 // Helpers of the GPU PDFIIM construction (cm_pdfiim_device).
 namespace {
+// count values of a device array in a new[] array (the caller's to release).
 template <class T>
-T *pd_new_copy(const std::vector<T> &v)
+int pd_take(T **h, const T *d, size_t count, hipStream_t s)
 {
-    T *p = new T[std::max<size_t>(v.size(), 1)];
-    std::copy(v.begin(), v.end(), p);
-    return p;
+    *h = new T[std::max<size_t>(count, 1)];
+    return copy_d2h(*h, d, count, s);
 }
 
 // Device buffers of one construction, freed on every exit.
+// Cut from a few chunks of doubling size: an allocation and its release cost
+// some 0.3 ms each, 12 ms of a 64^3 construction with one per buffer.
 struct PdBuffers {
     std::vector<void *> held;
     hipStream_t stream = nullptr;
+    char *at = nullptr;
+    size_t left = 0, chunk = (size_t)8 << 20;
     template <class T>
     int alloc(T **d, size_t count)
     {
-        CM_TRY(dev_alloc(d, count));
-        held.push_back((void *)*d);
+        const size_t bytes = (std::max<size_t>(count, 1) * sizeof(T) + 255) / 256 * 256;
+        if (bytes > left) {
+            chunk = std::max(2 * chunk, bytes);
+            at = nullptr;
+            left = 0;
+            CM_TRY(dev_alloc(&at, chunk));
+            held.push_back(at);
+            left = chunk;
+        }
+        *d = reinterpret_cast<T *>(at);
+        at += bytes;
+        left -= bytes;
         return CM_OK;
     }
     template <class T>
     int upload(T **d, const T *h, size_t count)
     {
         CM_TRY(alloc(d, count));
-        if (count) CM_HIP(hipMemcpyAsync(*d, h, count * sizeof(T), hipMemcpyHostToDevice, stream));
+        if (count) CM_TRY(copy_h2d(*d, h, count, stream));
+        return CM_OK;
+    }
+    // The transpose (ptr of n + 1, idx, val) of a list of n rows with nnz
+    // entries (ofs: the rows' first entries), columns below n.
+    template <class O>
+    int transpose(int n, int nnz, const O *ofs, const int *col, const double *val, int *ptr, int *idx, double *tval)
+    {
+        int *row, *ent, *key, *ent2;
+        CM_TRY(alloc(&row, 4 * (size_t)nnz));
+        ent = row + nnz, key = ent + nnz, ent2 = key + nnz;
+        int bits = 1;
+        while (bits < 31 && (1 << bits) < n) bits++;
+        k_pd_rows<O><<<long_grid(n), BS, 0, stream>>>(n, ofs, row, ent);
+        size_t tb = 0;
+        CM_HIP(hipcub::DeviceRadixSort::SortPairs(nullptr, tb, col, key, ent, ent2, nnz, 0, bits, stream));
+        char *tbuf;
+        CM_TRY(alloc(&tbuf, std::max<size_t>(tb, 1)));
+        CM_HIP(hipcub::DeviceRadixSort::SortPairs((void *)tbuf, tb, col, key, ent, ent2, nnz, 0, bits, stream));
+        k_pd_bounds<<<long_grid((long long)nnz + 1), BS, 0, stream>>>(n, nnz, key, ptr);
+        k_pd_permute<<<long_grid(nnz), BS, 0, stream>>>(nnz, ent2, row, val, idx, tval);
+        CM_HIP(hipGetLastError());
         return CM_OK;
     }
     ~PdBuffers()
@@ -3242,8 +3333,8 @@ int cm_system_get_x(cm_system h, double *x)
 {
     if (!h || !x) return fail(CM_ERR_ARG, "null argument");
     System &S = h->sys;
+    CM_TRY(copy_d2h(x, S.k64->x, (size_t)S.n, S.stream));
     CM_HIP(hipStreamSynchronize(S.stream));
-    CM_HIP(hipMemcpy(x, S.k64->x, (size_t)S.n * sizeof(double), hipMemcpyDeviceToHost));
     return CM_OK;
 }
 
@@ -3651,26 +3742,31 @@ int cm_pdfiim_device(int n, const double *Av, const int *Aj, const int *Ai, doub
     if (patt != 'B' && lfill > 1) return fail(CM_ERR_UNSUPPORTED, "patt 'L'/'U' need lfill == 1");
     // delete_last below an empty set is undefined in the reference
     if (warpsize != -1 && warpsize < 1) return fail(CM_ERR_ARG, "warpsize must be -1 or positive");
-    CM_TRY(check_csr(n, Ai, Aj));
-    std::vector<int> tp, tc;
-    std::vector<double> tv;
-    host_transpose(n, Ai, Aj, Av, tp, tc, tv);
+    if (const char *why = csr_ptr_problem(n, Ai, Aj)) return fail(CM_ERR_ARG, why);
     PdBuffers M;
     CM_HIP(hipStreamCreateWithFlags(&M.stream, hipStreamNonBlocking));
     const hipStream_t s = M.stream;
-    const long long nnz = Ai[n];
+    const int nnz = Ai[n];
     PdCsr A{}, At{};
     {
-        int *p, *c, *tpd, *tcd;
-        double *v, *tvd;
+        int *p, *c, *tp, *tc, *bad;
+        double *v, *tv;
         CM_TRY(M.upload(&p, Ai, (size_t)n + 1));
         CM_TRY(M.upload(&c, Aj, (size_t)nnz));
+        CM_TRY(M.alloc(&bad, 1));
+        CM_HIP(hipMemsetAsync(bad, 0, sizeof(int), s));
+        if (nnz) k_col_range<<<long_grid(nnz), BS, 0, s>>>(nnz, c, n, bad);
         CM_TRY(M.upload(&v, Av, (size_t)nnz));
-        CM_TRY(M.upload(&tpd, tp.data(), tp.size()));
-        CM_TRY(M.upload(&tcd, tc.data(), tc.size()));
-        CM_TRY(M.upload(&tvd, tv.data(), tv.size()));
+        int hbad = 0;
+        CM_HIP(hipMemcpyAsync(&hbad, bad, sizeof(int), hipMemcpyDeviceToHost, s));
+        CM_HIP(hipStreamSynchronize(s));  // before the columns index anything
+        if (hbad) return fail(CM_ERR_ARG, CSR_COL_RANGE);
+        CM_TRY(M.alloc(&tp, (size_t)n + 1));
+        CM_TRY(M.alloc(&tc, (size_t)nnz));
+        CM_TRY(M.alloc(&tv, (size_t)nnz));
+        CM_TRY(M.transpose(n, nnz, p, c, v, tp, tc, tv));
         A = PdCsr{p, c, v};
-        At = PdCsr{tpd, tcd, tvd};
+        At = PdCsr{tp, tc, tv};
     }
     const PdParams P{n, prefill, lfill, postfill, warpsize, ftol, std::max(1e-4, ftol), filttype, patt};
     int *gcnt, *hcnt, *flag;
@@ -3768,83 +3864,71 @@ int cm_pdfiim_device(int n, const double *Av, const int *Aj, const int *Ai, doub
     }
     (void)hipEventDestroy(e0);
     (void)hipEventDestroy(e1);
-    // counts and D back; packed offsets (row 0: the unit entry alone)
-    std::vector<int> gc(n, 1), hc(n, 1);
-    std::vector<double> dv(n);
-    if (nrows > 0) {
-        CM_HIP(hipMemcpyAsync(gc.data() + 1, gcnt + 1, (size_t)nrows * sizeof(int), hipMemcpyDeviceToHost, s));
-        CM_HIP(hipMemcpyAsync(hc.data() + 1, hcnt + 1, (size_t)nrows * sizeof(int), hipMemcpyDeviceToHost, s));
-        CM_HIP(hipMemcpyAsync(dv.data() + 1, dinv + 1, (size_t)nrows * sizeof(double), hipMemcpyDeviceToHost, s));
-        CM_HIP(hipStreamSynchronize(s));
+    // packed offsets (row 0: the unit entry alone), the packed lists, G by rows
+    // from its column lists (columns ascending in every row, the unit diagonal
+    // first)
+    long long *go, *ho;
+    CM_TRY(M.alloc(&go, 2 * ((size_t)n + 1)));
+    ho = go + n + 1;
+    k_pd_counts<<<long_grid(n), BS, 0, s>>>(n, gcnt, hcnt, A.val, dinv, go, ho);
+    {
+        size_t tb = 0;
+        CM_HIP(hipcub::DeviceScan::InclusiveSum(nullptr, tb, go + 1, go + 1, n, s));
+        char *tbuf;
+        CM_TRY(M.alloc(&tbuf, std::max<size_t>(tb, 1)));
+        CM_HIP(hipcub::DeviceScan::InclusiveSum((void *)tbuf, tb, go + 1, go + 1, n, s));
+        CM_HIP(hipcub::DeviceScan::InclusiveSum((void *)tbuf, tb, ho + 1, ho + 1, n, s));
     }
-    dv[0] = 1. / Av[0];  // PDFIIM/src/parPrec.cpp:132
-    std::vector<long long> go(n + 1, 0), ho(n + 1, 0);
-    for (int i = 0; i < n; i++) {
-        go[i + 1] = go[i] + gc[i];
-        ho[i + 1] = ho[i] + hc[i];
-    }
-    if (go[n] > INT_MAX || ho[n] > INT_MAX) return fail(CM_ERR_UNSUPPORTED, "factor has more than 2^31 entries");
-    std::vector<int> gpk(go[n]), hpk(ho[n]);
-    std::vector<double> gvk(go[n]), hvk(ho[n]);
-    gpk[0] = 0;
-    gvk[0] = 1.0;
-    hpk[0] = 0;
-    hvk[0] = 1.0;
+    long long gn = 0, hn = 0;
+    CM_HIP(hipMemcpyAsync(&gn, go + n, sizeof gn, hipMemcpyDeviceToHost, s));
+    CM_HIP(hipMemcpyAsync(&hn, ho + n, sizeof hn, hipMemcpyDeviceToHost, s));
+    CM_HIP(hipStreamSynchronize(s));
+    if (gn > INT_MAX || hn > INT_MAX) return fail(CM_ERR_UNSUPPORTED, "factor has more than 2^31 entries");
+    int *gci, *hpi, *gpi, *gpj, *hptr;
+    double *gcv, *hpv, *gpv;
+    CM_TRY(M.alloc(&gci, (size_t)gn));
+    CM_TRY(M.alloc(&gcv, (size_t)gn));
+    CM_TRY(M.alloc(&hpi, (size_t)hn));
+    CM_TRY(M.alloc(&hpv, (size_t)hn));
+    CM_TRY(M.alloc(&hptr, (size_t)n + 1));
+    CM_TRY(M.alloc(&gpi, (size_t)n + 1));
+    CM_TRY(M.alloc(&gpj, (size_t)gn));
+    CM_TRY(M.alloc(&gpv, (size_t)gn));
+    k_pd_finish<<<long_grid((long long)n + 1), BS, 0, s>>>(n, ho, hptr, gci, gcv, hpi, hpv);
     if (nrows > 0) {
-        long long *god, *hod;
-        int *gpd, *hpd;
-        double *gvd, *hvd;
-        CM_TRY(M.upload(&god, go.data(), go.size()));
-        CM_TRY(M.upload(&hod, ho.data(), ho.size()));
-        CM_TRY(M.alloc(&gpd, (size_t)go[n]));
-        CM_TRY(M.alloc(&hpd, (size_t)ho[n]));
-        CM_TRY(M.alloc(&gvd, (size_t)go[n]));
-        CM_TRY(M.alloc(&hvd, (size_t)ho[n]));
         const int g1 = (int)std::min<long long>((nrows + BS - 1) / BS, 8192);
-        k_pd_pack<<<g1, BS, 0, s>>>(nrows, nullptr, OUT1, gcnt, god, gi1, gv1, gpd, gvd);
-        k_pd_pack<<<g1, BS, 0, s>>>(nrows, nullptr, OUT1, hcnt, hod, hi1, hv1, hpd, hvd);
+        k_pd_pack<<<g1, BS, 0, s>>>(nrows, nullptr, OUT1, gcnt, go, gi1, gv1, gci, gcv);
+        k_pd_pack<<<g1, BS, 0, s>>>(nrows, nullptr, OUT1, hcnt, ho, hi1, hv1, hpi, hpv);
         if (n2) {  // the tier-2 rows overwrite their (stale) tier-1 slots' packed places
             const int g2 = (int)std::min<long long>((n2 + BS - 1) / BS, 8192);
-            k_pd_pack<<<g2, BS, 0, s>>>(n2, rows2d, OUT2, gcnt, god, gi2, gv2, gpd, gvd);
-            k_pd_pack<<<g2, BS, 0, s>>>(n2, rows2d, OUT2, hcnt, hod, hi2, hv2, hpd, hvd);
+            k_pd_pack<<<g2, BS, 0, s>>>(n2, rows2d, OUT2, gcnt, go, gi2, gv2, gci, gcv);
+            k_pd_pack<<<g2, BS, 0, s>>>(n2, rows2d, OUT2, hcnt, ho, hi2, hv2, hpi, hpv);
         }
         if (n3) {  // and the tier-3 rows theirs
             const int g3 = (int)std::min<long long>((n3 + BS - 1) / BS, 8192);
-            k_pd_pack<<<g3, BS, 0, s>>>(n3, rows3d, OUT3, gcnt, god, gi3, gv3, gpd, gvd);
-            k_pd_pack<<<g3, BS, 0, s>>>(n3, rows3d, OUT3, hcnt, hod, hi3, hv3, hpd, hvd);
+            k_pd_pack<<<g3, BS, 0, s>>>(n3, rows3d, OUT3, gcnt, go, gi3, gv3, gci, gcv);
+            k_pd_pack<<<g3, BS, 0, s>>>(n3, rows3d, OUT3, hcnt, ho, hi3, hv3, hpi, hpv);
         }
         CM_HIP(hipGetLastError());
-        const size_t g0 = (size_t)go[1], h0 = (size_t)ho[1];
-        CM_HIP(hipMemcpyAsync(gpk.data() + g0, gpd + g0, (go[n] - g0) * sizeof(int), hipMemcpyDeviceToHost, s));
-        CM_HIP(hipMemcpyAsync(gvk.data() + g0, gvd + g0, (go[n] - g0) * sizeof(double), hipMemcpyDeviceToHost, s));
-        CM_HIP(hipMemcpyAsync(hpk.data() + h0, hpd + h0, (ho[n] - h0) * sizeof(int), hipMemcpyDeviceToHost, s));
-        CM_HIP(hipMemcpyAsync(hvk.data() + h0, hvd + h0, (ho[n] - h0) * sizeof(double), hipMemcpyDeviceToHost, s));
-        CM_HIP(hipStreamSynchronize(s));
     }
-    // H rows are the packed row lists; G by rows from its column lists
-    // (columns ascending in every row, the unit diagonal first)
-    std::vector<int> hptr(n + 1), gptr(n + 1, 0);
-    for (int i = 0; i <= n; i++) hptr[i] = (int)ho[i];
-    for (long long k = 0; k < go[n]; k++) gptr[gpk[k] + 1]++;
-    for (int i = 0; i < n; i++) gptr[i + 1] += gptr[i];
-    std::vector<int> gj(go[n]);
-    std::vector<double> gvv(go[n]);
-    {
-        std::vector<int> fill(gptr.begin(), gptr.end() - 1);
-        for (int i = 0; i < n; i++)
-            for (long long k = go[i]; k < go[i + 1]; k++) {
-                const int q = fill[gpk[k]]++;
-                gj[q] = i;
-                gvv[q] = gvk[k];
-            }
+    CM_TRY(M.transpose(n, (int)gn, go, gci, gcv, gpi, gpj, gpv));
+    // straight into the caller's arrays
+    int rc = pd_take(Gindi, gpi, (size_t)n + 1, s);
+    if (rc == CM_OK) rc = pd_take(Gindj, gpj, (size_t)gn, s);
+    if (rc == CM_OK) rc = pd_take(Gval, gpv, (size_t)gn, s);
+    if (rc == CM_OK) rc = pd_take(Hindi, hptr, (size_t)n + 1, s);
+    if (rc == CM_OK) rc = pd_take(Hindj, hpi, (size_t)hn, s);
+    if (rc == CM_OK) rc = pd_take(Hval, hpv, (size_t)hn, s);
+    if (rc == CM_OK) rc = pd_take(IDv, dinv, (size_t)n, s);
+    if (rc == CM_OK && hipStreamSynchronize(s) != hipSuccess) rc = fail(CM_ERR_HIP, "factors could not be copied back");
+    if (rc != CM_OK) {
+        (void)hipStreamSynchronize(s);
+        delete[] *Gindi, delete[] *Gindj, delete[] *Hindi, delete[] *Hindj;
+        delete[] *Gval, delete[] *Hval, delete[] *IDv;
+        *Gval = *Hval = *IDv = nullptr;
+        *Gindj = *Gindi = *Hindj = *Hindi = nullptr;
+        return rc;
     }
-    *Gindi = pd_new_copy(gptr);
-    *Gindj = pd_new_copy(gj);
-    *Gval = pd_new_copy(gvv);
-    *Hindi = pd_new_copy(hptr);
-    *Hindj = pd_new_copy(hpk);
-    *Hval = pd_new_copy(hvk);
-    *IDv = pd_new_copy(dv);
     if (device_ms) *device_ms = ms_total;
     return CM_OK;
 }

@@ -469,6 +469,75 @@ __global__ __launch_bounds__(BS) void k_pd_pack(int nrows, const int *__restrict
     }
 }
 
+// ---- transposes and packed offsets of the construction
+//
+// A transpose is a stable sort of the entries by column (cub's radix sort on
+// (column, entry)), which leaves every column's entries in row order, as the
+// host's counting pass over the rows does; the row pointers are the columns'
+// first places in the sorted keys.
+
+// row[k], ent[k] of every entry k of a list of n rows (ofs: first entries).
+template <class O>
+__global__ __launch_bounds__(BS) void k_pd_rows(int n, const O *__restrict__ ofs, int *__restrict__ row,
+                                                int *__restrict__ ent)
+{
+    for (int i = blockIdx.x * BS + threadIdx.x; i < n; i += gridDim.x * BS)
+        for (long long k = ofs[i]; k < (long long)ofs[i + 1]; k++) {
+            row[k] = i;
+            ent[k] = (int)k;
+        }
+}
+
+// ptr[c] = first place of a key >= c among the sorted keys, c = 0 .. n.
+__global__ __launch_bounds__(BS) void k_pd_bounds(int n, int nnz, const int *__restrict__ key, int *__restrict__ ptr)
+{
+    for (int k = blockIdx.x * BS + threadIdx.x; k <= nnz; k += gridDim.x * BS) {
+        const int lo = k ? key[k - 1] + 1 : 0, hi = k < nnz ? key[k] : n;
+        for (int c = lo; c <= hi; c++) ptr[c] = k;
+    }
+}
+
+// The transposed entries in sorted order: their rows and values.
+__global__ __launch_bounds__(BS) void k_pd_permute(int nnz, const int *__restrict__ ent, const int *__restrict__ row,
+                                                   const double *__restrict__ val, int *__restrict__ tidx,
+                                                   double *__restrict__ tval)
+{
+    for (int q = blockIdx.x * BS + threadIdx.x; q < nnz; q += gridDim.x * BS) {
+        const int k = ent[q];
+        tidx[q] = row[k];
+        tval[q] = val[k];
+    }
+}
+
+// Row 0 of the factors is the unit entry alone, with D(0) = 1 / A(0, first)
+// (PDFIIM/src/parPrec.cpp:132); the counts as 64-bit numbers behind a zero,
+// for the scans that make them offsets.
+__global__ __launch_bounds__(BS) void k_pd_counts(int n, const int *__restrict__ gcnt, const int *__restrict__ hcnt,
+                                                  const double *__restrict__ av, double *__restrict__ dinv,
+                                                  long long *__restrict__ go, long long *__restrict__ ho)
+{
+    const int t0 = blockIdx.x * BS + threadIdx.x;
+    if (t0 == 0) {
+        dinv[0] = 1. / av[0];
+        go[0] = ho[0] = 0;
+    }
+    for (int i = t0; i < n; i += gridDim.x * BS) {
+        go[i + 1] = i ? gcnt[i] : 1;
+        ho[i + 1] = i ? hcnt[i] : 1;
+    }
+}
+
+__global__ __launch_bounds__(BS) void k_pd_finish(int n, const long long *__restrict__ ho, int *__restrict__ hptr,
+                                                  int *gi, double *gv, int *hi, double *hv)
+{
+    const int t0 = blockIdx.x * BS + threadIdx.x;
+    if (t0 == 0) {
+        gi[0] = hi[0] = 0;
+        gv[0] = hv[0] = 1.0;
+    }
+    for (int i = t0; i <= n; i += gridDim.x * BS) hptr[i] = (int)ho[i];
+}
+
 }  // namespace cm
 
 namespace cm {
