@@ -27,6 +27,7 @@
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
+#include <chrono>
 #include <climits>
 #include <cmath>
 #include <condition_variable>
@@ -343,6 +344,12 @@ struct SlotIndex {
     }
 };
 
+// The longest row and the most entries in RS_GROUP consecutive rows of a CSR
+// structure, -1: not known yet.
+struct RowSpread {
+    int longest = -1, group = -1;
+};
+
 // Index arrays of a matrix's diagonal copy (spmv_dia), shared like
 // SlotIndex: the diagonal offsets, for every diagonal element the CSR
 // position of its entry (-1: none, stored as 0), and the CSR remainder of
@@ -351,6 +358,7 @@ struct DiaIndex {
     int n = 0, ldn = 0, nd = 0;  // ldn: diagonal stride, n rounded up to DIA_ALIGN
     long long nrem = 0;
     std::vector<int> hoff;  // the offsets on the host, ascending
+    mutable RowSpread spread;  // of the remainder (resident solves)
     int *off = nullptr, *dsrc = nullptr, *rptr = nullptr, *rcol = nullptr, *rsrc = nullptr;
     // Rows whose remainder is longer than SHORT_MAX, for the block products:
     // lpos[row] = their index q (0..nlong-1), -1 for the other rows.  Their
@@ -420,6 +428,7 @@ struct DevCsr {
     bool use16 = false;       // low-precision copy: products through spmv_vl16
     V *val = nullptr;
     float *rowscale = nullptr;
+    mutable RowSpread spread;          // (resident solves)
     std::shared_ptr<SlotIndex> slots;  // slot-major index (shared by the copies), if built
     V *sval = nullptr;                 // this copy's values in slot-major order, if built
     bool use_slot = false;             // products through spmv_slot
@@ -490,6 +499,7 @@ struct DevCsr {
         rowscale = nullptr;
         slots.reset();
         dia.reset();
+        spread = RowSpread();
         use_slot = slot16 = use_dia = block_dia = false;
     }
     ~DevCsr() { release(); }
@@ -1136,6 +1146,244 @@ struct HostSys {
     const double *Uv;
 };
 
+// CUs promised to resident grids, per device: a grid waits for all its
+// workgroups, so grids whose workgroups together exceed the CUs are not in
+// flight at once (from several threads, or a server's workers).  Each
+// workgroup counts as a CU.
+class ResidentGate {
+  public:
+    static ResidentGate &get()
+    {
+        static ResidentGate g;
+        return g;
+    }
+    static constexpr int MAX_DEV = 64;
+    // The first of the nc sizes wgs[] that fits the CUs not promised, waiting
+    // up to WAIT for one to fit; its index, or -1 (the caller's launched
+    // passes need no promise).
+    static constexpr std::chrono::milliseconds WAIT{3};
+    int acquire(int dev, const int *wgs, int nc, int cus)
+    {
+        if (dev < 0 || dev >= MAX_DEV) return -1;
+        int got = -1;
+        auto fits = [&] {
+            for (got = 0; got < nc; got++)
+                if (used[dev] + wgs[got] <= cus) return true;
+            got = -1;
+            return false;
+        };
+        std::unique_lock<std::mutex> lk(mu);
+        if (!cv.wait_for(lk, WAIT, fits)) return -1;
+        used[dev] += wgs[got];
+        return got;
+    }
+    void release(int dev, int wgs)
+    {
+        {
+            std::lock_guard<std::mutex> lk(mu);
+            used[dev] -= wgs;
+        }
+        cv.notify_all();
+    }
+
+  private:
+    std::mutex mu;
+    std::condition_variable cv;
+    int used[MAX_DEV] = {};
+};
+
+// A launch shape of a resident solve (threads and rows per thread of its
+// workgroups, and the workgroups of one column), and the shapes a solve can
+// take, the preferred one first.
+struct RsShape {
+    int bsz, rows, wgs;
+};
+struct RsPlan {
+    RsShape s[4];
+    int count = 0;
+};
+
+// What a solver keeps for its resident solves (cm_resident.hpp), made on
+// first use: reduction slots and control words on the device, the columns'
+// results in pinned memory.
+template <class T, class VA, class VF>
+struct RsRunner {
+    double *slots = nullptr;
+    RsCtl *ctl = nullptr;
+    RsTable<T, VA, VF> *args = nullptr;
+    SolveState *out = nullptr;
+    int slot_cols = 0, skip = 0;
+    ~RsRunner()
+    {
+        (void)hipFree(slots);
+        (void)hipFree(ctl);
+        (void)hipFree(args);
+        if (out) (void)hipHostFree(out);
+    }
+    static int cus(int *dev)
+    {
+        int c = 0;
+        if (hipGetDevice(dev) != hipSuccess) return 0;
+        if (hipDeviceGetAttribute(&c, hipDeviceAttributeMultiprocessorCount, *dev) != hipSuccess) return 0;
+        return std::min(c, RS_WGS);
+    }
+    // Matrix m for workgroups of `rows` rows, bsz of them per step: its
+    // diagonal copy where that is built (whichever format the launched
+    // products use) and its x windows fit, else CSR.
+    template <class V>
+    static RsMat<V> mat(const DevCsr<V> &m, int bsz, int rows)
+    {
+        RsMat<V> q;
+        std::memset(&q, 0, sizeof q);
+        q.rowscale = m.rowscale;
+        if (m.dia && m.dval && rs_windows(m.dia->hoff, bsz, rows, q)) {
+            const DiaIndex &D = *m.dia;
+            q.nd = D.nd;
+            q.ldn = D.ldn;
+            q.dval = m.dval;
+            q.ptr = D.rptr;
+            q.col = D.rcol;
+            q.val = m.rval;
+        } else {
+            q.ns = 0;
+            q.ptr = m.ptr;
+            q.col = m.col;
+            q.val = m.val;
+        }
+        return q;
+    }
+    // The longest row and the most entries in RS_GROUP consecutive rows of
+    // what mat() leaves in CSR, found on the device once per matrix.
+    template <class V>
+    int spread(const DevCsr<V> &m, int bsz, int rows, hipStream_t stream, RowSpread &w)
+    {
+        const RsMat<V> q = mat(m, bsz, rows);
+        w = RowSpread{0, 0};
+        if (!q.ptr) return CM_OK;
+        RowSpread &keep = q.nd ? m.dia->spread : m.spread;
+        if (keep.longest < 0) {
+            CM_TRY(ensure(1));
+            int *d = reinterpret_cast<int *>(ctl);
+            CM_HIP(hipMemsetAsync(d, 0, sizeof(RowSpread), stream));
+            k_row_spread<<<(m.n + RS_GROUP - 1) / RS_GROUP, RS_GROUP, 0, stream>>>(m.n, q.ptr, d);
+            CM_HIP(hipGetLastError());
+            CM_HIP(hipMemcpyAsync(out, d, sizeof(RowSpread), hipMemcpyDeviceToHost, stream));
+            CM_HIP(hipStreamSynchronize(stream));
+            std::memcpy(&keep, out, sizeof(RowSpread));
+        }
+        w = keep;
+        return CM_OK;
+    }
+    int ensure(int nc)
+    {
+        if (nc > slot_cols) {
+            (void)hipFree(slots);
+            slots = nullptr;
+            slot_cols = 0;
+            CM_TRY(dev_alloc(&slots, (size_t)nc * RS_SETS * RS_K * RS_WGS));
+            slot_cols = nc;
+        }
+        if (!ctl) CM_TRY(dev_alloc(&ctl, 1));
+        if (!args) CM_TRY(dev_alloc(&args, 1));
+        if (!out) CM_HIP(hipHostMalloc((void **)&out, RS_COLS * sizeof(SolveState), hipHostMallocDefault));
+        return CM_OK;
+    }
+    // The shapes whose grids for nc columns fit the device, one workgroup per
+    // CU.  Small workgroups run a pass faster (46656 rows, FP64: 28 us on 512
+    // rows, 37 on 1024 and 58 on 2048; FP32: 30, 31 and 38), large ones leave
+    // CUs to other solves: smallest first for a lone column (`all`) and in
+    // FP64; a block in FP32 first the smallest that takes at most half of the
+    // CUs, else the largest (a burst of 24 requests on six systems took 9 ms
+    // instead of 13 with the smallest first, where the grids had to wait for
+    // each other).
+    // Entries in CSR are gathered past the L2s, RS_PER * bsz at a time, and
+    // added by their row's thread.  Launched / resident us per pass of FP64,
+    // by these gather steps of the three products: 62 / 40 at 256^2 rows on
+    // 1.8 steps, 102 / 73 at 512^2 on 3.7, 73 / 72 at 64^3 on 7, 158 / 154 at
+    // 724^2 on 7.4 (FP32 112 / 85); 90 / 2160 at 90^2 rows of 370 entries, on
+    // 53 steps whose long rows are summed serially.
+    int plan(int n, int nc, bool all, const DevCsr<VA> &A, const DevCsr<VF> &H, const DevCsr<VF> &G,
+             hipStream_t stream, RsPlan &p)
+    {
+        p.count = 0;
+        if (n < 1 || n > RS_MAX_ROWS || nc > RS_COLS) return CM_OK;
+        int dev = 0;
+        const int cap = cus(&dev);
+        for (const RsShape &s : {RsShape{256, 1, 0}, RsShape{512, 1, 0}, RsShape{512, 2, 0}, RsShape{512, 4, 0}}) {
+            const int rows = s.bsz * s.rows;
+            RsShape f = s;
+            f.wgs = (n + rows - 1) / rows;
+            if ((long long)f.wgs * nc > cap) continue;
+            RowSpread w[3];
+            CM_TRY(spread(A, s.bsz, rows, stream, w[0]));
+            CM_TRY(spread(H, s.bsz, rows, stream, w[1]));
+            CM_TRY(spread(G, s.bsz, rows, stream, w[2]));
+            double steps = 0.0, serial = 0.0;
+            for (const RowSpread &q : w) {
+                steps += (double)q.group * rows / RS_GROUP / (RS_PER * s.bsz);
+                serial += q.longest;
+            }
+            if (steps > RS_CSR_STEPS * (1.0 + (double)n / RS_MAX_ROWS) || serial > RS_CSR_ROW) continue;
+            p.s[p.count++] = f;
+            if (all) return CM_OK;
+        }
+        if (p.count == 0 || sizeof(T) == 8) return CM_OK;
+        int first = 0;
+        while (first < p.count && p.s[first].wgs * nc > cap / 2) first++;
+        if (first == p.count) {  // every shape takes more than half
+            std::reverse(p.s, p.s + p.count);
+            return CM_OK;
+        }
+        p.count -= first;
+        for (int q = 0; q < p.count; q++) p.s[q] = p.s[q + first];
+        return CM_OK;
+    }
+    // Runs the columns of a (its matrices and buffers filled in here).  ran:
+    // all of them did; else x is as it was in those that did not.
+    int run(RsArgs<T, VA, VF> &a, const DevCsr<VA> &A, const DevCsr<VF> &H, const DevCsr<VF> &G, const RsPlan &p,
+            hipStream_t stream, bool &ran)
+    {
+        ran = false;
+        const int nc = a.ncols;
+        int dev = 0, wgs[4];
+        const int cap = cus(&dev);
+        CM_TRY(ensure(nc));
+        std::memset(out, 0, RS_COLS * sizeof(SolveState));
+        if (skip > 0) {
+            skip--;
+            return CM_OK;
+        }
+        for (int q = 0; q < p.count; q++) wgs[q] = p.s[q].wgs * nc;
+        const int pick = ResidentGate::get().acquire(dev, wgs, p.count, cap);
+        if (pick < 0) return CM_OK;
+        struct Held {
+            int dev, wgs;
+            ~Held() { ResidentGate::get().release(dev, wgs); }
+        } held{dev, wgs[pick]};
+        const RsShape &s = p.s[pick];
+        const int rows = s.bsz * s.rows;
+        a.A = mat(A, s.bsz, rows);
+        a.H = mat(H, s.bsz, rows);
+        a.G = mat(G, s.bsz, rows);
+        a.slots = slots;
+        a.ctl = ctl;
+        a.out = out;
+        const dim3 grid(s.wgs, nc);
+        k_rs_prep<T, VA, VF><<<vec_grid(a.n), BS, 0, stream>>>(a, args);
+        if (s.bsz == 256) k_rs_solve<T, VA, VF, 256, 1><<<grid, 256, 0, stream>>>(args);
+        else if (s.rows == 1) k_rs_solve<T, VA, VF, 512, 1><<<grid, 512, 0, stream>>>(args);
+        else if (s.rows == 2) k_rs_solve<T, VA, VF, 512, 2><<<grid, 512, 0, stream>>>(args);
+        else k_rs_solve<T, VA, VF, 512, 4><<<grid, 512, 0, stream>>>(args);
+        CM_HIP(hipGetLastError());
+        CM_HIP(hipStreamSynchronize(stream));
+        ran = true;
+        for (int c = 0; c < nc; c++) ran = ran && out[c].done;
+        // a device too busy for the grid: the next solves do not try
+        if (!ran) skip = RS_SKIP;
+        return CM_OK;
+    }
+};
+
 // The BiCGSTAB core for vectors of type T, A values of type VA and factor
 // values of type VF.
 template <class T, class VA, class VF>
@@ -1164,9 +1412,7 @@ struct Krylov {
     hipGraphExec_t g1 = nullptr, gN = nullptr;
     TrsvCtl *trsv_ctl = nullptr;  // control words of an apply's two triangular solves (modes I, J)
     bool resident = false;       // whole solves in one launch (tuned systems; run_resident)
-    double *rs_slots = nullptr;  // reduction slots and control words of the resident solve (first use)
-    RsCtl *rs_ctl = nullptr;
-    RsArgs<T, VA, VF> *rs_args = nullptr;
+    RsRunner<T, VA, VF> rs;
 
     void drop_graphs()
     {
@@ -1184,9 +1430,6 @@ struct Krylov {
         (void)hipFree(partials);
         (void)hipFree(trace);
         (void)hipFree(trsv_ctl);
-        (void)hipFree(rs_slots);
-        (void)hipFree(rs_ctl);
-        (void)hipFree(rs_args);
         (void)hipFree(st);
         if (hst) (void)hipHostFree(hst);
         for (auto &e : ev)
@@ -1525,60 +1768,23 @@ struct Krylov {
         return CM_OK;
     }
 
-    // Matrix m for workgroups of `rows` rows, bsz of them per step: its
-    // diagonal copy where that is built (whichever format the launched
-    // products use) and its x windows fit, else CSR.
-    template <class V>
-    static RsMat<V> rs_mat(const DevCsr<V> &m, int bsz, int rows)
-    {
-        RsMat<V> q;
-        std::memset(&q, 0, sizeof q);
-        q.rowscale = m.rowscale;
-        if (m.dia && m.dval && rs_windows(m.dia->hoff, bsz, rows, q)) {
-            const DiaIndex &D = *m.dia;
-            q.nd = D.nd;
-            q.ldn = D.ldn;
-            q.dval = m.dval;
-            q.ptr = D.rptr;
-            q.col = D.rcol;
-            q.val = m.rval;
-        } else {
-            q.ns = 0;
-            q.ptr = m.ptr;
-            q.col = m.col;
-            q.val = m.val;
-        }
-        return q;
-    }
-
-    // The whole solve in one resident launch (cm_resident.hpp), in apply mode
-    // E on systems that were tuned (or come from a one-shot call), which leave
-    // the summation order to the engine.  Per pass it took, against the
-    // captured launches, 19 / 45 us at 100^2, 26 / 54 us at 45^3, 42 / 73 us
-    // at 64^3 and 86 / 115 us at 79^3 rows (FP64; FP32 50 / 91 us at 79^3),
-    // up to RS_MAX_ROWS, the most rows whose state the registers hold.  With a
-    // matrix in CSR the gathers go past the L2s entry by entry: 26 / 55 us at
-    // 100^2 but 72 / 73 us at 64^3, so beyond 65536 rows every matrix has to
-    // be in diagonals.  ran = false: not taken, or the grid could not be
-    // resident; x is untouched and the caller enqueues passes.  Launches being
-    // bracketed by profiling events are the passes', so a profiled solve does
-    // not come here.
+    // The whole solve in one resident launch (RsRunner), in apply mode E on
+    // systems that were tuned (or come from a one-shot call), which leave the
+    // summation order to the engine.  Per pass it took, against the captured
+    // launches, 19 / 45 us at 100^2, 26 / 54 us at 45^3, 42 / 73 us at 64^3 and
+    // 86 / 115 us at 79^3 rows (FP64; FP32 50 / 91 us at 79^3), up to
+    // RS_MAX_ROWS, the most rows whose state the registers hold.  ran = false:
+    // not taken, or the grid could not be resident; x is untouched and the
+    // caller enqueues passes.  Launches being bracketed by profiling events
+    // are the passes', so a profiled solve does not come here.
     int run_resident(double tol, int NMAX, int info_in, int trace_cap, bool zero_start, SolveState &fin, bool &ran)
     {
         ran = false;
-        if (!resident || prof.on || (variant == 2 && mode != 'E') || n > RS_MAX_ROWS) return CM_OK;
-        int dev = 0, cus = 0;
-        CM_HIP(hipGetDevice(&dev));
-        CM_HIP(hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev));
-        const int bsz = n <= RS_WGS * 256 ? 256 : 512;
-        const int rows = n <= RS_WGS * 512 ? 1 : n <= RS_WGS * 1024 ? 2 : 4;
-        const int grid = (n + bsz * rows - 1) / (bsz * rows);
-        if (grid > std::min(cus, RS_WGS)) return CM_OK;
-        if (!rs_slots) CM_TRY(dev_alloc(&rs_slots, (size_t)RS_SETS * RS_K * RS_WGS));
-        if (!rs_ctl) CM_TRY(dev_alloc(&rs_ctl, 1));
-        if (!rs_args) CM_TRY(dev_alloc(&rs_args, 1));
-        SolveState *out = &hst[1];
-        std::memset(out, 0, sizeof *out);
+        if (!resident || prof.on || (variant == 2 && mode != 'E')) return CM_OK;
+        RsPlan plan;
+        CM_TRY(rs.plan(n, 1, true, A, sym ? GT : H, G, stream, plan));
+        if (plan.count == 0) return CM_OK;
+        CM_TRY(ensure_trace(trace_cap));
         RsArgs<T, VA, VF> a;
         std::memset(&a, 0, sizeof a);
         a.n = n;
@@ -1588,31 +1794,18 @@ struct Krylov {
         a.info_in = info_in;
         a.zero_start = zero_start ? 1 : 0;
         a.trace_cap = trace_cap;
-        a.tol = tol;
+        a.trace = trace_cap > 0 ? trace : nullptr;
+        a.stride = 1;
+        a.ncols = 1;
+        a.tol[0] = tol;
         a.eps = eps;
-        a.A = rs_mat(A, bsz, bsz * rows);
-        a.H = rs_mat(sym ? GT : H, bsz, bsz * rows);
-        a.G = rs_mat(G, bsz, bsz * rows);
-        if (n > RS_WGS * 256 && !(a.A.nd && a.H.nd && a.G.nd)) return CM_OK;
         a.idv = idv;
         a.b = b;
         a.x = x;
         T *ex[6] = {p, tm, pc, s, t1, sc};
         for (int q = 0; q < 6; q++) a.ex[q] = ex[q];
-        CM_TRY(ensure_trace(trace_cap));
-        a.trace = trace_cap > 0 ? trace : nullptr;
-        a.slots = rs_slots;
-        a.ctl = rs_ctl;
-        a.out = out;
-        k_rs_prep<T, VA, VF><<<vec_grid(n), BS, 0, stream>>>(a, rs_args);
-        if (bsz == 256) k_rs_solve<T, VA, VF, 256, 1><<<grid, 256, 0, stream>>>(rs_args);
-        else if (rows == 1) k_rs_solve<T, VA, VF, 512, 1><<<grid, 512, 0, stream>>>(rs_args);
-        else if (rows == 2) k_rs_solve<T, VA, VF, 512, 2><<<grid, 512, 0, stream>>>(rs_args);
-        else k_rs_solve<T, VA, VF, 512, 4><<<grid, 512, 0, stream>>>(rs_args);
-        CM_HIP(hipGetLastError());
-        CM_HIP(hipStreamSynchronize(stream));
-        fin = *out;
-        ran = fin.done != 0;
+        CM_TRY(rs.run(a, A, sym ? GT : H, G, plan, stream, ran));
+        fin = rs.out[0];
         return CM_OK;
     }
 
@@ -2031,6 +2224,7 @@ struct BlockKrylov {
     bool racc_short = false;  // a product was refused: racc smaller than it needs (nothing launched)
     hipEvent_t ev[2] = {nullptr, nullptr};
     bool use_graph = true;
+    RsRunner<T, VA, VF> rs;
     hipGraphExec_t g1 = nullptr, gN = nullptr;  // one pass, GRAPH_PASSES passes
 
     ~BlockKrylov()
@@ -2383,6 +2577,65 @@ struct BlockKrylov {
         return CM_OK;
     }
 
+    // The active columns in resident launches, each column on workgroups of
+    // its own with its own scalars and exit: all columns at once where their
+    // workgroups fit the CUs, in FP32 else in two halves (FP64 halves took
+    // longer than the launched passes).  A launched pass is some 16 kernels
+    // whatever the width.  Per pass, launched / here: 46656 rows, FP32 63 / 31
+    // us for 2 columns, 91 / 34 for 5, 92 / 42 for 8, 106 / 77 for 14 (halves),
+    // FP64 61 / 29, 88 / 45, 90 / 82; 6859 rows, FP32 64-72 / 30.  active: the
+    // columns to run, on return those still to run (none when ran); fin: the
+    // states of those that did.
+    int run_resident(double tol, int NMAX, int *active, const double *col_tol, bool zero_start, SolveState *fin,
+                     bool &ran)
+    {
+        ran = false;
+        std::vector<int> cols;
+        for (int j = 0; j < ncols; j++)
+            if (active[j]) cols.push_back(j);
+        const int nc = (int)cols.size();
+        RsPlan plan;
+        int per = nc;
+        if (nc == 0) return CM_OK;
+        CM_TRY(rs.plan(n, per, false, *A, *Hm, *G, stream, plan));
+        if (plan.count == 0 && sizeof(T) == 4 && nc > 1) {
+            per = (nc + 1) / 2;
+            CM_TRY(rs.plan(n, per, false, *A, *Hm, *G, stream, plan));
+        }
+        if (plan.count == 0) return CM_OK;
+        for (int c0 = 0; c0 < nc; c0 += per) {
+            RsArgs<T, VA, VF> a;
+            std::memset(&a, 0, sizeof a);
+            a.n = n;
+            a.nmax = NMAX;
+            a.variant = variant;
+            a.maxmsteps = max_div_steps(variant, n);
+            a.zero_start = zero_start ? 1 : 0;
+            a.stride = KB;
+            a.ncols = std::min(per, nc - c0);
+            for (int c = 0; c < a.ncols; c++) {
+                a.col[c] = cols[c0 + c];
+                a.tol[c] = col_tol ? col_tol[cols[c0 + c]] : tol;
+            }
+            a.eps = eps;
+            a.idv = idv;
+            a.b = b;
+            a.x = x;
+            T *ex[6] = {p, tm, pc, s, t, sc};
+            for (int q = 0; q < 6; q++) a.ex[q] = ex[q];
+            bool ok;
+            CM_TRY(rs.run(a, *A, *Hm, *G, plan, stream, ok));
+            for (int c = 0; c < a.ncols; c++) {
+                if (!rs.out[c].done) continue;
+                fin[cols[c0 + c]] = rs.out[c];
+                active[cols[c0 + c]] = 0;
+            }
+            if (!ok) return CM_OK;
+        }
+        ran = true;
+        return CM_OK;
+    }
+
     void setup_from_x() { spmm(*A, bA, x, BEpiSetup<T>{r, r0, p, b}, st); }
 
     void setup_zero()
@@ -2581,10 +2834,18 @@ struct BlockSolver : BlockBase {
 
     int solve64(double tol, int NMAX, double *resval, int *iter, int *info) override
     {
-        CM_TRY(b64.begin(tol, NMAX, nullptr));
-        b64.setup_from_x();
-        SolveState fin[KB];
-        CM_TRY(b64.run(NMAX, fin));
+        SolveState fin[KB], rest[KB];
+        std::vector<int> act(KB, 0);
+        for (int j = 0; j < ncols; j++) act[j] = 1;
+        bool ran;
+        CM_TRY(b64.run_resident(tol, NMAX, act.data(), nullptr, false, fin, ran));
+        if (!ran) {  // the columns left (a launched column that is done keeps its x)
+            CM_TRY(b64.begin(tol, NMAX, act.data()));
+            b64.setup_from_x();
+            CM_TRY(b64.run(NMAX, rest));
+            for (int j = 0; j < ncols; j++)
+                if (act[j]) fin[j] = rest[j];
+        }
         for (int j = 0; j < ncols; j++) {
             resval[j] = fin[j].rc / fin[j].ro;
             iter[j] = fin[j].iter;
@@ -2645,10 +2906,15 @@ struct BlockSolver : BlockBase {
                 loose[j] = act[j] && itol[j] > inner_tol;
                 if (act[j]) act[j] = 1;
             }
-            CM_TRY(bi.begin(inner_tol, NMAX, act.data(), itol.data()));
-            bi.setup_zero();
             SolveState fin[KB];
-            CM_TRY(bi.run(NMAX, fin));
+            std::vector<int> todo(act);
+            bool ran;
+            CM_TRY(bi.run_resident(inner_tol, NMAX, todo.data(), itol.data(), true, fin, ran));
+            if (!ran) {
+                CM_TRY(bi.begin(inner_tol, NMAX, act.data(), itol.data()));
+                bi.setup_zero();
+                CM_TRY(bi.run(NMAX, fin));
+            }
             int most = 0;
             for (int j = 0; j < ncols; j++)
                 if (act[j]) most = std::max(most, fin[j].ntrace);

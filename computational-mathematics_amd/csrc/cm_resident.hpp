@@ -22,6 +22,10 @@
 // barrier with cache invalidation 2.5-6 us and a kernel boundary 3.5 us.
 // A result that equals the marker bit for bit is published as another NaN.
 //
+// Columns.  The right-hand sides of a block are columns of the grid (gridDim
+// y): each has its own workgroups, exchanged vectors, reduction slots,
+// scalars and exits, and they meet only on arrival.
+//
 // The two reductions of a pass (alpha; omega) are all-to-all exchanges of the
 // workgroups' partial sums, added in workgroup order by every workgroup, so
 // all of them compute the same scalars and take the same exits.  They also
@@ -46,7 +50,11 @@ constexpr int RS_MAX_ROWS = RS_WGS * 1024 * 2;
 constexpr int RS_PER = 8;                  // staged entries per thread and step
 constexpr int RS_STEPS = 16;               // window steps at most (half of them with 1024 threads)
 constexpr int RS_SPINS = 1 << 20;          // loads of one entry before a wait gives up (about a second)
-constexpr long long RS_JOIN_TICKS = 20000;  // 100 MHz ticks the grid may take to arrive (200 us)
+constexpr int RS_GROUP = 256;              // rows over which the spread of CSR entries is taken
+constexpr double RS_CSR_STEPS = 4.0;       // gather steps of the three products' CSR entries (twice that at the most rows)
+constexpr double RS_CSR_ROW = 256.0;       // entries of the three products' longest CSR rows
+constexpr int RS_SKIP = 16;                // launched solves after a grid that did not arrive
+constexpr long long RS_JOIN_TICKS = 1000000;  // 100 MHz ticks the grid may take to arrive (10 ms)
 constexpr int RS_K = 4;                    // sums per reduction
 constexpr int RS_SETS = 5;                 // reduction slots: setup, alpha and omega of even and odd passes
 
@@ -167,19 +175,37 @@ static bool rs_windows(const std::vector<int> &off, int bsz, int rows, RsMat<V> 
     return true;
 }
 
+// Column k of the launch (blockIdx.y) is column col[k] of b and x, which hold
+// `stride` columns interleaved, and solves to tol[k].
+constexpr int RS_COLS = 16;
 template <class T, class VA, class VF>
 struct RsArgs {
-    int n, nmax, variant, maxmsteps, info_in, zero_start, trace_cap, pad;
-    double tol, eps;
-    double *trace;  // device
+    int n, nmax, variant, maxmsteps, info_in, zero_start, trace_cap, stride, ncols;
+    int col[RS_COLS];
+    double tol[RS_COLS], eps;
+    double *trace;  // device; first column
     RsMat<VF> H, G;
     RsMat<VA> A;
     const T *idv, *b;
     T *x;
-    T *ex[6];  // exchanged vectors: p, H p, M p, s, H s, M s
-    double *slots;                     // RS_SETS x RS_K x RS_WGS
+    T *ex[6];         // exchanged vectors of ncols x n: p, H p, M p, s, H s, M s
+    double *slots;    // ncols x RS_SETS x RS_K x RS_WGS
     RsCtl *ctl;
-    SolveState *out;  // pinned host memory
+    SolveState *out;  // pinned host memory, one per column of the launch
+};
+
+// What differs between the columns of a launch.
+template <class T>
+struct RsCol {
+    double tol, *slots, *trace;
+    T *ex[6], *x;
+    const T *b;
+    SolveState *out;
+};
+template <class T, class VA, class VF>
+struct RsTable {
+    RsArgs<T, VA, VF> a;
+    RsCol<T> c[RS_COLS];
 };
 
 // The arguments lie in device memory and are read through the scalar cache
@@ -187,23 +213,53 @@ struct RsArgs {
 template <class X>
 using RsConst = const __attribute__((address_space(4))) X *;
 
+// The longest row and the most entries in RS_GROUP consecutive rows, out[0]
+// and out[1] (0 before); a workgroup per group.
+__global__ __launch_bounds__(RS_GROUP) void k_row_spread(int n, const int *ptr, int *out)
+{
+    const int r0 = blockIdx.x * RS_GROUP, i = r0 + threadIdx.x;
+    int len = i < n ? ptr[i + 1] - ptr[i] : 0;
+    for (int d = WAVE / 2; d > 0; d /= 2) len = max(len, __shfl_xor(len, d, WAVE));
+    if (threadIdx.x % WAVE == 0) atomicMax(out, len);
+    if (threadIdx.x == 0) atomicMax(out + 1, ptr[min(r0 + RS_GROUP, n)] - ptr[r0]);
+}
+
 // Markers into the exchanged vectors and reduction slots, control words 0,
-// and the arguments to where the solve reads them.
+// and the arguments to where the solve reads them (every column's pointers
+// ready: computed in the solve they made a pass 1.5% slower).
 template <class T, class VA, class VF>
-__global__ __launch_bounds__(BS) void k_rs_prep(RsArgs<T, VA, VF> a, RsArgs<T, VA, VF> *to)
+__global__ __launch_bounds__(BS) void k_rs_prep(RsArgs<T, VA, VF> a, RsTable<T, VA, VF> *to)
 {
     const int t0 = blockIdx.x * BS + threadIdx.x, st = gridDim.x * BS;
     using U = typename RsBits<T>::U;
-    for (int i = t0; i < a.n; i += st) {
+    for (int i = t0; i < a.n * a.ncols; i += st) {
 #pragma unroll
         for (int e = 0; e < 6; e++) reinterpret_cast<U *>(a.ex[e])[i] = RsBits<T>::MARK;
     }
-    for (int i = t0; i < RS_SETS * RS_K * RS_WGS; i += st)
+    for (int i = t0; i < a.ncols * RS_SETS * RS_K * RS_WGS; i += st)
         reinterpret_cast<unsigned long long *>(a.slots)[i] = RsBits<double>::MARK;
     if (t0 == 0) {
         a.ctl->join = 0;
         a.ctl->verdict = 0;
-        *to = a;
+        to->a = a;
+    }
+    if (t0 < a.ncols) {
+        RsCol<T> c;
+        int col = 0;
+#pragma unroll
+        for (int k = 0; k < RS_COLS; k++)
+            if (k == t0) {
+                c.tol = a.tol[k];
+                col = a.col[k];
+            }
+        c.slots = a.slots + (size_t)t0 * RS_SETS * RS_K * RS_WGS;
+        c.trace = t0 == 0 ? a.trace : nullptr;
+#pragma unroll
+        for (int e = 0; e < 6; e++) c.ex[e] = a.ex[e] + (size_t)t0 * a.n;
+        c.x = a.x + col;
+        c.b = a.b + col;
+        c.out = a.out + t0;
+        to->c[t0] = c;
     }
 }
 
@@ -484,6 +540,7 @@ __device__ __forceinline__ void rs_allsum(double (&v)[RS_K], double *slots, int 
 // Arrival of the grid; true when every workgroup is running.
 __device__ __forceinline__ bool rs_join(RsCtl *c, int *sh)
 {
+    const unsigned all = gridDim.x * gridDim.y;
     if (threadIdx.x == 0) {
         constexpr unsigned CLOSED = 0x80000000u;
         unsigned verdict = 2;
@@ -491,11 +548,11 @@ __device__ __forceinline__ bool rs_join(RsCtl *c, int *sh)
         if (!(q & CLOSED)) {
             if (q == 0) {
                 const long long t0 = wall_clock64();
-                while (__hip_atomic_load(&c->join, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) < gridDim.x &&
+                while (__hip_atomic_load(&c->join, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) < all &&
                        wall_clock64() - t0 < RS_JOIN_TICKS) {
                 }
                 const unsigned f = __hip_atomic_fetch_or(&c->join, CLOSED, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-                verdict = f == gridDim.x ? 1u : 2u;
+                verdict = f == all ? 1u : 2u;
                 __hip_atomic_store(&c->verdict, verdict, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
             } else {
                 for (int spin = 0; spin < RS_SPINS; spin++) {
@@ -520,9 +577,10 @@ __device__ __forceinline__ bool rs_join(RsCtl *c, int *sh)
 // reduction carries anyway, r0 . s - omega (r0 . t), where r0 . s is what
 // rounding leaves of 0; this saves an exchange of 2 us per pass.
 template <class T, class VA, class VF, int BSZ, int R>
-__global__ __launch_bounds__(BSZ) void k_rs_solve(const RsArgs<T, VA, VF> *args)
+__global__ __launch_bounds__(BSZ) void k_rs_solve(const RsTable<T, VA, VF> *args)
 {
-    auto g = (RsConst<RsArgs<T, VA, VF>>)args;
+    auto g = (RsConst<RsArgs<T, VA, VF>>)&args->a;
+    auto c = (RsConst<RsCol<T>>)&args->c[blockIdx.y];
     using Acc = typename std::conditional<std::is_same<T, double>::value, double, float>::type;
     __shared__ Acc prod[RS_PER * BSZ];
     __shared__ T win[rs_steps(BSZ) * BSZ];
@@ -540,8 +598,11 @@ __global__ __launch_bounds__(BSZ) void k_rs_solve(const RsArgs<T, VA, VF> *args)
         x[q] = r[q] = dv[q] = r0[q] = p[q] = v[q] = w[q] = (T)0;
         if (i < n) {
             dv[q] = rs_glob(g->idv)[i];
-            r[q] = rs_glob(g->b)[i];
-            if (!g->zero_start) x[q] = rs_glob(g->x)[i];
+            r[q] = rs_glob(c->b)[(size_t)i * g->stride];
+            if (!g->zero_start) {  // the initial residual gathers x
+                x[q] = rs_glob(c->x)[(size_t)i * g->stride];
+                rs_put(rs_glob(c->ex[5]) + i, x[q]);
+            }
         }
     }
     // diagonals held in registers: a 7-point matrix's and its PDFIIM factors'
@@ -567,12 +628,13 @@ __global__ __launch_bounds__(BSZ) void k_rs_solve(const RsArgs<T, VA, VF> *args)
     for (;;) {
         // the matrices' tables are read again in every step: kept across
         // steps they would take the registers that hold the values
-        asm volatile("" : "+s"(g));
+        asm volatile("" : "+s"(g), "+s"(c));
         Acc y[R];
-        const T *src = rs_glob(g->x);
+        const T *src = rs_glob(c->ex[5]);
         if (step != 6) {
-            T *const ex[3] = {rs_glob(step == 2 ? g->ex[0] : g->ex[3]), rs_glob(step == 2 ? g->ex[1] : g->ex[4]),
-                              rs_glob(step == 2 ? g->ex[2] : g->ex[5])};
+            T *const ex[3] = {rs_glob(step == 2 ? c->ex[0] : c->ex[3]),
+                              rs_glob(step == 2 ? c->ex[1] : c->ex[4]),
+                              rs_glob(step == 2 ? c->ex[2] : c->ex[5])};
             rs_rows<T, VF, Acc, BSZ, R, 17>(&g->H, dh, tile, lo[0], hi[0], n, row0, ex[0], win, prod, dead, y);
             rs_ahead<VF, Acc, BSZ, R>(&g->G, lo[1], hi[1], n, row0, tile);
 #pragma unroll
@@ -629,7 +691,7 @@ __global__ __launch_bounds__(BSZ) void k_rs_solve(const RsArgs<T, VA, VF> *args)
                 sm[0] += (double)r[q] * (double)r[q];
             }
         }
-        rs_allsum<BSZ>(sm, rs_glob(g->slots), set, red[set], dead);
+        rs_allsum<BSZ>(sm, rs_glob(c->slots), set, red[set], dead);
         if (rs_uni(*dead)) return;
         if (step == 2) {
             alpha = m1 / sm[0];
@@ -649,13 +711,13 @@ __global__ __launch_bounds__(BSZ) void k_rs_solve(const RsArgs<T, VA, VF> *args)
                 x[q] = x[q] + al * w[q];
                 r[q] = r[q] + na * v[q];  // s
                 if (i < n) {
-                    rs_put(rs_glob(g->ex[3]) + i, r[q]);
+                    rs_put(rs_glob(c->ex[3]) + i, r[q]);
 #pragma unroll
-                    for (int e = 0; e < 3; e++) rs_put_bits(rs_glob(g->ex[e]) + i, RsBits<T>::MARK);
+                    for (int e = 0; e < 3; e++) rs_put_bits(rs_glob(c->ex[e]) + i, RsBits<T>::MARK);
                 }
             }
             if (tid < RS_K)
-                rs_put_bits(rs_glob(g->slots) + ((size_t)(3 + (par ^ 1)) * RS_K + tid) * RS_WGS + blockIdx.x,
+                rs_put_bits(rs_glob(c->slots) + ((size_t)(3 + (par ^ 1)) * RS_K + tid) * RS_WGS + blockIdx.x,
                             RsBits<double>::MARK);
             step = 5;
             continue;
@@ -674,7 +736,7 @@ __global__ __launch_bounds__(BSZ) void k_rs_solve(const RsArgs<T, VA, VF> *args)
             else stag = 0;
             const double prc = rc;
             rc = rn;
-            if (g->trace && ntrace < g->trace_cap && blockIdx.x == 0 && tid == 0) g->trace[ntrace] = rc;
+            if (c->trace && ntrace < g->trace_cap && blockIdx.x == 0 && tid == 0) c->trace[ntrace] = rc;
             ntrace++;
             if (prc < rc) msteps++;
             else msteps = 0;
@@ -686,7 +748,7 @@ __global__ __launch_bounds__(BSZ) void k_rs_solve(const RsArgs<T, VA, VF> *args)
                 info = 2;
                 break;
             }
-            if (rc < g->tol * ro) {
+            if (rc < c->tol * ro) {
                 info = 0;
                 break;
             }
@@ -716,15 +778,15 @@ __global__ __launch_bounds__(BSZ) void k_rs_solve(const RsArgs<T, VA, VF> *args)
         for (int q = 0; q < R; q++) {
             const int i = row0 + q * BSZ + tid;
             if (i < n) {
-                rs_put(rs_glob(g->ex[0]) + i, p[q]);
-                if (step == 5)
+                rs_put(rs_glob(c->ex[0]) + i, p[q]);
+                if (step == 5 || !g->zero_start)
 #pragma unroll
-                    for (int e = 3; e < 6; e++) rs_put_bits(rs_glob(g->ex[e]) + i, RsBits<T>::MARK);
+                    for (int e = 3; e < 6; e++) rs_put_bits(rs_glob(c->ex[e]) + i, RsBits<T>::MARK);
             }
         }
         if (step == 5) {
             if (tid < RS_K)
-                rs_put_bits(rs_glob(g->slots) + ((size_t)(1 + par) * RS_K + tid) * RS_WGS + blockIdx.x, RsBits<double>::MARK);
+                rs_put_bits(rs_glob(c->slots) + ((size_t)(1 + par) * RS_K + tid) * RS_WGS + blockIdx.x, RsBits<double>::MARK);
             par ^= 1;
         }
         step = 2;
@@ -732,10 +794,10 @@ __global__ __launch_bounds__(BSZ) void k_rs_solve(const RsArgs<T, VA, VF> *args)
 #pragma unroll
     for (int q = 0; q < R; q++) {
         const int i = row0 + q * BSZ + tid;
-        if (i < n && (g->nmax > 0 || g->zero_start)) rs_glob(g->x)[i] = x[q];
+        if (i < n && (g->nmax > 0 || g->zero_start)) rs_glob(c->x)[(size_t)i * g->stride] = x[q];
     }
     if (blockIdx.x == 0 && tid == 0) {
-        SolveState *o = g->out;
+        SolveState *o = c->out;
         o->ro = ro;
         o->rc = rc;
         o->iter = iter;
