@@ -1771,8 +1771,8 @@ struct Krylov {
     // The whole solve in one resident launch (RsRunner), in apply mode E on
     // systems that were tuned (or come from a one-shot call), which leave the
     // summation order to the engine.  Per pass it took, against the captured
-    // launches, 19 / 45 us at 100^2, 26 / 54 us at 45^3, 42 / 73 us at 64^3 and
-    // 86 / 115 us at 79^3 rows (FP64; FP32 50 / 91 us at 79^3), up to
+    // launches, 18 / 45 us at 100^2, 26 / 54 us at 45^3, 40 / 73 us at 64^3 and
+    // 86 / 115 us at 79^3 rows (FP64; FP32 47 / 91 us at 79^3), up to
     // RS_MAX_ROWS, the most rows whose state the registers hold.  ran = false:
     // not taken, or the grid could not be resident; x is untouched and the
     // caller enqueues passes.  Launches being bracketed by profiling events

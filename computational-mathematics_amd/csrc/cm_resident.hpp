@@ -6,10 +6,13 @@
 // is bound by launches, kernel boundaries and dependent loads, not by memory.
 // Here every workgroup owns a fixed range of rows, and each thread keeps its
 // R rows' x, r (then s), r0, p, v and M p (then M s), and their values on the
-// matrices' diagonals, in registers for the whole solve.  FP64, per pass: 19
-// us at 100^2 rows (45 launched), 26 us at 45^3 (54), 42 us at 64^3 (73), 86
-// us at 79^3 (115).  What bounds it is the chain of eight exchanges of about
-// 2.1 us; beyond 131072 rows (FP64) the values held spill or are read again.
+// matrices' diagonals, in registers for the whole solve.  FP64, per pass: 18
+// us at 100^2 rows (45 launched), 26 us at 45^3 (54), 40 us at 64^3 (73), 86
+// us at 79^3 (115).  What bounds it is the chain of eight exchanges: of the
+// pass at 100^2 rows the gathers of its six products are 6.5 us, the two
+// reductions 5.5, the sums over the diagonals 2, the rest LDS writes, barriers
+// and stores.  Beyond 131072 rows (FP64) the values held spill or are read
+// again.
 //
 // Exchange.  Only the vectors that other rows gather go through memory (p,
 // H p, M p and s, H s, M s).  Each entry is its own arrival flag: the buffers
@@ -356,6 +359,28 @@ __device__ __forceinline__ void rs_hold(RsConst<RsMat<V>> m, int n, int row0, V 
     }
 }
 
+// The first NW window steps and the entries fetched ahead, gathered together.
+template <class T, class V, class Acc, int BSZ, int R, int NW>
+__device__ __forceinline__ void rs_first(RsConst<RsMat<V>> m, const RsTile<Acc, R> &f, bool rest, int n, int row0,
+                                         const T *x, T *win, Acc *prod, volatile int *dead)
+{
+    constexpr int NR = rs_nr<Acc, R>();
+    const int tid = (int)threadIdx.x, ns = m->ns;
+    int j[NW + NR];
+    T xv[NW + NR];
+#pragma unroll
+    for (int q = 0; q < NW; q++) j[q] = rs_window(m, q, n, row0);
+#pragma unroll
+    for (int q = 0; q < NR; q++) j[NW + q] = f.j[q];
+    rs_gather<T, NW + NR>(x, j, xv, dead);
+#pragma unroll
+    for (int q = 0; q < NW; q++)
+        if (q < ns) win[q * BSZ + tid] = xv[q];
+    if (rest)
+#pragma unroll
+        for (int q = 0; q < NR; q++) prod[q * BSZ + tid] = f.ev[q] * (Acc)xv[NW + q];
+}
+
 // Row sums y of m x for the workgroup's R * BSZ rows from row0 on (row q *
 // BSZ + thread of them in y[q]).  The part of x that the diagonals touch is a
 // few windows (diagonals whose offsets lie closer than the workgroup's rows
@@ -373,19 +398,9 @@ __device__ __forceinline__ void rs_rows(RsConst<RsMat<V>> m, const V (&dv)[R][ND
 #pragma clang fp contract(off)
     constexpr int NR = rs_nr<Acc, R>();
     const int tid = (int)threadIdx.x, nd = m->nd, ns = m->ns;
-    int j[RS_NW + NR];
-    T xv[RS_NW + NR];
-#pragma unroll
-    for (int q = 0; q < RS_NW; q++) j[q] = rs_window(m, q, n, row0);
-#pragma unroll
-    for (int q = 0; q < NR; q++) j[RS_NW + q] = f.j[q];
-    rs_gather<T, RS_NW + NR>(x, j, xv, dead);
-#pragma unroll
-    for (int q = 0; q < RS_NW; q++)
-        if (q < ns) win[q * BSZ + tid] = xv[q];
-    if (re > rs)
-#pragma unroll
-        for (int q = 0; q < NR; q++) prod[q * BSZ + tid] = f.ev[q] * (Acc)xv[RS_NW + q];
+    // fewer loads in the chain where few windows are read (no second copy with 4 rows per thread: spills)
+    if (R < 4 && ns <= RS_NW / 2) rs_first<T, V, Acc, BSZ, R, RS_NW / 2>(m, f, re > rs, n, row0, x, win, prod, dead);
+    else rs_first<T, V, Acc, BSZ, R, RS_NW>(m, f, re > rs, n, row0, x, win, prod, dead);
     for (int s0 = RS_NW; s0 < ns; s0 += RS_NW) {
         int j2[RS_NW];
         T x2[RS_NW];
@@ -398,13 +413,40 @@ __device__ __forceinline__ void rs_rows(RsConst<RsMat<V>> m, const V (&dv)[R][ND
     __syncthreads();
 #pragma unroll
     for (int q = 0; q < R; q++) y[q] = 0;
+    if constexpr (R >= 4) {  // no registers left for more than one at a time
 #pragma unroll
-    for (int d = 0; d < ND; d++)
-        if (d < nd) {
-            const int w = m->wpos[d] + tid;
+        for (int d = 0; d < ND; d++)
+            if (d < nd) {
+                const int w = m->wpos[d] + tid;
 #pragma unroll
-            for (int q = 0; q < R; q++) y[q] += dia_val<V, Acc>(dv[q][d]) * (Acc)win[w + q * BSZ];
-        }
+                for (int q = 0; q < R; q++) y[q] += dia_val<V, Acc>(dv[q][d]) * (Acc)win[w + q * BSZ];
+            }
+    } else {
+        // DH diagonals at a time: their positions, their x, then the sums in
+        // order.  One by one each waited for its position and its x, 60 cycles
+        // a diagonal; with this and the shorter gather of few windows a pass
+        // took 18.3 us instead of 19.2 at 100^2 rows, 25.9 (27.5) at 45^3,
+        // 40.3 (43.5) at 64^3 and in FP32 24.8 (27.9) and 32.1 (34.7).
+        constexpr int DH = R * sizeof(Acc) <= 8 ? 6 : 4;
+#pragma unroll
+        for (int d0 = 0; d0 < ND; d0 += DH)
+            if (d0 < nd) {
+                T xd[R][DH];
+#pragma unroll
+                for (int d = 0; d < DH; d++)
+#pragma unroll
+                    for (int q = 0; q < R; q++)
+                        if (d0 + d < ND) xd[q][d] = win[m->wpos[d0 + d] + tid + q * BSZ];
+#pragma unroll
+                for (int d = 0; d < DH; d++)
+                    if (d0 + d < ND)
+#pragma unroll
+                        for (int q = 0; q < R; q++) {
+                            const Acc t = dia_val<V, Acc>(dv[q][d0 + d]) * (Acc)xd[q][d];
+                            y[q] += d0 + d < nd ? t : (Acc)0;  // y, a sum begun at 0, is never -0
+                        }
+            }
+    }
     for (int d0 = ND; d0 < nd; d0 += RS_DC) {  // diagonals not held
         V v[R][RS_DC];
 #pragma unroll
@@ -590,7 +632,7 @@ __global__ __launch_bounds__(BSZ) void k_rs_solve(const RsTable<T, VA, VF> *args
     if (!rs_join(g->ctl, &sh_join)) return;
     volatile int *dead = &sh_dead;
     const int n = g->n, tid = threadIdx.x;
-    const int row0 = (int)blockIdx.x * R * BSZ;
+    int row0 = (int)blockIdx.x * R * BSZ;
     T x[R], r[R], r0[R], p[R], v[R], w[R], dv[R];  // w: M p, then M s
 #pragma unroll
     for (int q = 0; q < R; q++) {
@@ -629,6 +671,7 @@ __global__ __launch_bounds__(BSZ) void k_rs_solve(const RsTable<T, VA, VF> *args
         // the matrices' tables are read again in every step: kept across
         // steps they would take the registers that hold the values
         asm volatile("" : "+s"(g), "+s"(c));
+        if constexpr (R == 2 && sizeof(T) == 8) asm volatile("" : "+s"(row0));  // and the rows' addresses
         Acc y[R];
         const T *src = rs_glob(c->ex[5]);
         if (step != 6) {
