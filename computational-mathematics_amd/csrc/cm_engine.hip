@@ -159,6 +159,7 @@ class Stager {
             copy(buf[b], (const char *)src + off, len);
             CM_HIP(hipMemcpyAsync((char *)dst + off, buf[b], len, hipMemcpyHostToDevice, s));
             CM_HIP(hipEventCreateWithFlags(&ev[b], hipEventDisableTiming));  // on the stream's (current) device
+            on[b] = s;
             CM_HIP(hipEventRecord(ev[b], s));
             off += len;
         }
@@ -186,6 +187,7 @@ class Stager {
             len[q] = std::min(CHUNK / 4, bytes - asked);
             CM_HIP(hipMemcpyAsync(buf[b[q]], (const char *)src + asked, len[q], hipMemcpyDeviceToHost, s));
             CM_HIP(hipEventCreateWithFlags(&ev[b[q]], hipEventDisableTiming));
+            on[b[q]] = s;
             CM_HIP(hipEventRecord(ev[b[q]], s));
             asked += len[q];
             n++;
@@ -200,6 +202,17 @@ class Stager {
             n--;
         }
         return CM_OK;
+    }
+
+    // No event recorded on s is left: called before s is captured or
+    // destroyed.  Waiting for an event looks at the stream it was recorded on:
+    // one that is gone by then, or that another thread captures, made the wait
+    // of a later transfer fail.
+    void settle(hipStream_t s)
+    {
+        std::lock_guard<std::mutex> lk(mu);
+        for (int b = 0; b < NBUF; b++)
+            if (ev[b] && on[b] == s) (void)drain(b);
     }
 
   private:
@@ -222,6 +235,7 @@ class Stager {
     std::mutex mu;  // one transfer at a time
     char *buf[NBUF] = {};
     hipEvent_t ev[NBUF] = {};  // recorded behind each chunk's last copy
+    hipStream_t on[NBUF] = {};  // on this stream
     int next = 0;              // the chunk filled next
     struct Job {
         char *d;
@@ -1723,6 +1737,7 @@ struct Krylov {
         const bool prof_on = prof.on;  // captured passes carry no timing events
         const int pass = prof.pass;
         prof.on = false;
+        Stager::get().settle(stream);
         CM_HIP(hipStreamBeginCapture(stream, hipStreamCaptureModeThreadLocal));
         for (int i = 0; i < passes; i++) enqueue_iteration();
         const hipError_t cerr = hipStreamEndCapture(stream, &graph);
@@ -2529,6 +2544,7 @@ struct BlockKrylov {
     int capture(hipGraphExec_t &out, int passes)
     {
         hipGraph_t graph = nullptr;
+        Stager::get().settle(stream);
         CM_HIP(hipStreamBeginCapture(stream, hipStreamCaptureModeThreadLocal));
         for (int i = 0; i < passes; i++) enqueue_iteration();
         CM_HIP(hipStreamEndCapture(stream, &graph));
@@ -3090,7 +3106,10 @@ struct System {
         k64.reset();
         (void)hipFree(ost);
         if (host_ost) (void)hipHostFree(host_ost);
-        if (stream) (void)hipStreamDestroy(stream);
+        if (stream) {
+            Stager::get().settle(stream);
+            (void)hipStreamDestroy(stream);
+        }
     }
 };
 
@@ -3513,7 +3532,10 @@ struct PdBuffers {
     {
         if (stream) (void)hipStreamSynchronize(stream);
         for (void *q : held) (void)hipFree(q);
-        if (stream) (void)hipStreamDestroy(stream);
+        if (stream) {
+            Stager::get().settle(stream);
+            (void)hipStreamDestroy(stream);
+        }
     }
 };
 }  // namespace

@@ -487,7 +487,10 @@ int cm_server_destroy(cm_server h)
     S.cv_work.notify_all();
     S.cv_done.notify_all();
     for (auto &t : S.workers) t.join();
-    for (auto s : S.streams) (void)hipStreamDestroy(s);
+    for (auto s : S.streams) {
+        Stager::get().settle(s);
+        (void)hipStreamDestroy(s);
+    }
     for (double *p : S.pin)
         if (p) (void)hipHostFree(p);
     delete h;
