@@ -4031,7 +4031,14 @@ int cm_pdfiim_device(int n, const double *Av, const int *Aj, const int *Ai, doub
     // delete_last below an empty set is undefined in the reference
     if (warpsize != -1 && warpsize < 1) return fail(CM_ERR_ARG, "warpsize must be -1 or positive");
     if (const char *why = csr_ptr_problem(n, Ai, Aj)) return fail(CM_ERR_ARG, why);
+    // few columns are checked here: the flag's way to the host takes 35 us
+    const bool host_check = Ai[n] <= 1 << 16;
+    if (host_check)
+        if (const char *why = csr_problem(n, Ai, Aj)) return fail(CM_ERR_ARG, why);
     PdBuffers M;
+    // a small construction's buffers take about 1 KB per row (a first chunk of
+    // 16 MB for them cost 0.1-0.4 ms now and then)
+    M.chunk = std::min(M.chunk, std::max((size_t)n << 10, (size_t)1 << 19));
     CM_HIP(hipStreamCreateWithFlags(&M.stream, hipStreamNonBlocking));
     const hipStream_t s = M.stream;
     const int nnz = Ai[n];
@@ -4041,14 +4048,16 @@ int cm_pdfiim_device(int n, const double *Av, const int *Aj, const int *Ai, doub
         double *v, *tv;
         CM_TRY(M.upload(&p, Ai, (size_t)n + 1));
         CM_TRY(M.upload(&c, Aj, (size_t)nnz));
-        CM_TRY(M.alloc(&bad, 1));
-        CM_HIP(hipMemsetAsync(bad, 0, sizeof(int), s));
-        if (nnz) k_col_range<<<long_grid(nnz), BS, 0, s>>>(nnz, c, n, bad);
         CM_TRY(M.upload(&v, Av, (size_t)nnz));
-        int hbad = 0;
-        CM_HIP(hipMemcpyAsync(&hbad, bad, sizeof(int), hipMemcpyDeviceToHost, s));
-        CM_HIP(hipStreamSynchronize(s));  // before the columns index anything
-        if (hbad) return fail(CM_ERR_ARG, CSR_COL_RANGE);
+        if (!host_check) {
+            CM_TRY(M.alloc(&bad, 1));
+            CM_HIP(hipMemsetAsync(bad, 0, sizeof(int), s));
+            k_col_range<<<long_grid(nnz), BS, 0, s>>>(nnz, c, n, bad);
+            int hbad = 0;
+            CM_HIP(hipMemcpyAsync(&hbad, bad, sizeof(int), hipMemcpyDeviceToHost, s));
+            CM_HIP(hipStreamSynchronize(s));  // before the columns index anything
+            if (hbad) return fail(CM_ERR_ARG, CSR_COL_RANGE);
+        }
         CM_TRY(M.alloc(&tp, (size_t)n + 1));
         CM_TRY(M.alloc(&tc, (size_t)nnz));
         CM_TRY(M.alloc(&tv, (size_t)nnz));
@@ -4167,21 +4176,24 @@ int cm_pdfiim_device(int n, const double *Av, const int *Aj, const int *Ai, doub
         CM_HIP(hipcub::DeviceScan::InclusiveSum((void *)tbuf, tb, go + 1, go + 1, n, s));
         CM_HIP(hipcub::DeviceScan::InclusiveSum((void *)tbuf, tb, ho + 1, ho + 1, n, s));
     }
-    long long gn = 0, hn = 0;
-    CM_HIP(hipMemcpyAsync(&gn, go + n, sizeof gn, hipMemcpyDeviceToHost, s));
-    CM_HIP(hipMemcpyAsync(&hn, ho + n, sizeof hn, hipMemcpyDeviceToHost, s));
+    long long totals[2] = {0, 0};  // go[n], ho[n]
+    CM_HIP(hipMemcpy2DAsync(totals, sizeof totals[0], go + n, ((size_t)n + 1) * sizeof totals[0], sizeof totals[0], 2,
+                            hipMemcpyDeviceToHost, s));
     CM_HIP(hipStreamSynchronize(s));
+    const long long gn = totals[0], hn = totals[1];
     if (gn > INT_MAX || hn > INT_MAX) return fail(CM_ERR_UNSUPPORTED, "factor has more than 2^31 entries");
-    int *gci, *hpi, *gpi, *gpj, *hptr;
-    double *gcv, *hpv, *gpv;
+    int *gci;
+    double *gcv;
     CM_TRY(M.alloc(&gci, (size_t)gn));
     CM_TRY(M.alloc(&gcv, (size_t)gn));
-    CM_TRY(M.alloc(&hpi, (size_t)hn));
-    CM_TRY(M.alloc(&hpv, (size_t)hn));
-    CM_TRY(M.alloc(&hptr, (size_t)n + 1));
-    CM_TRY(M.alloc(&gpi, (size_t)n + 1));
-    CM_TRY(M.alloc(&gpj, (size_t)gn));
-    CM_TRY(M.alloc(&gpv, (size_t)gn));
+    // the results side by side, so that small ones leave in one copy
+    double *gpv;
+    const size_t ints = 2 * ((size_t)n + 1) + (size_t)gn + (size_t)hn;
+    const size_t out_bytes = (size_t)(gn + hn) * sizeof(double) + ints * sizeof(int);
+    CM_TRY(M.alloc(reinterpret_cast<char **>(&gpv), out_bytes));
+    double *const hpv = gpv + gn;
+    int *const gpi = reinterpret_cast<int *>(hpv + hn), *const hptr = gpi + n + 1, *const gpj = hptr + n + 1,
+              *const hpi = gpj + gn;
     k_pd_finish<<<long_grid((long long)n + 1), BS, 0, s>>>(n, ho, hptr, gci, gcv, hpi, hpv);
     if (nrows > 0) {
         const int g1 = (int)std::min<long long>((nrows + BS - 1) / BS, 8192);
@@ -4200,6 +4212,33 @@ int cm_pdfiim_device(int n, const double *Av, const int *Aj, const int *Ai, doub
         CM_HIP(hipGetLastError());
     }
     CM_TRY(M.transpose(n, (int)gn, go, gci, gcv, gpi, gpj, gpv));
+    if (out_bytes < Stager::MIN_BYTES) {  // seven small copies took 80 us more than these two
+        std::vector<char> h(out_bytes);
+        CM_HIP(hipMemcpyAsync(h.data(), gpv, out_bytes, hipMemcpyDeviceToHost, s));
+        *IDv = new double[std::max(n, 1)];
+        if (hipMemcpyAsync(*IDv, dinv, (size_t)n * sizeof(double), hipMemcpyDeviceToHost, s) != hipSuccess ||
+            hipStreamSynchronize(s) != hipSuccess) {
+            (void)hipStreamSynchronize(s);
+            delete[] *IDv;
+            *IDv = nullptr;
+            return fail(CM_ERR_HIP, "factors could not be copied back");
+        }
+        const char *at = h.data();
+        auto take = [&at](auto **d, size_t count) {
+            using V = typename std::remove_reference<decltype(**d)>::type;
+            *d = new V[std::max<size_t>(count, 1)];
+            std::memcpy(*d, at, count * sizeof(V));
+            at += count * sizeof(V);
+        };
+        take(Gval, (size_t)gn);
+        take(Hval, (size_t)hn);
+        take(Gindi, (size_t)n + 1);
+        take(Hindi, (size_t)n + 1);
+        take(Gindj, (size_t)gn);
+        take(Hindj, (size_t)hn);
+        if (device_ms) *device_ms = ms_total;
+        return CM_OK;
+    }
     // straight into the caller's arrays
     int rc = pd_take(Gindi, gpi, (size_t)n + 1, s);
     if (rc == CM_OK) rc = pd_take(Gindj, gpj, (size_t)gn, s);
