@@ -13,6 +13,9 @@
 // the counter passes the item count, and every solve ends by NMAX, so the
 // grid always drains.
 //
+// Systems of at most BT_ROWS rows run in k_batch_small, which keeps the
+// vectors in LDS and registers and streams the matrices through LDS; the rest
+// of this comment is k_batch_solve, for larger ones.
 // Per workgroup: SpMV rows go to groups of LPR lanes (xor-shuffle sums inside
 // the group); vector updates stride over the rows; dot products and norms
 // are summed in a fixed order (per-thread, wave shuffles, then the waves in

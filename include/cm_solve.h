@@ -144,7 +144,8 @@ int cm_system_block_get(cm_system sys, double *X);
  * default) or launched kernel by kernel (off); the results are identical.
  * cm_system_graphs covers the single-RHS solves (which launch kernel by
  * kernel anyway while cm_system_profile brackets launches), and
- * cm_system_block_graphs the block solves. */
+ * cm_system_block_graphs the block solves.  Solves that run in one launch
+ * (tuned systems and blocks of at most 524288 rows) do so in both cases. */
 int cm_system_graphs(cm_system sys, int on);
 int cm_system_block_graphs(cm_system sys, int on);
 /* Persistent batched solves: nitems right-hand sides of small resident
@@ -157,7 +158,8 @@ int cm_system_block_graphs(cm_system sys, int on);
  * while its true residual is above tol (at most 4 cycles, NMAX passes in
  * total); 0 is the reference loop.  Apply mode E; per-item resval, iter,
  * info as in cm_system_solve.  Suited to systems whose solve is launch-bound
- * (up to some 10^4-10^5 rows); work vectors take 9 n doubles per resident
+ * (up to some 10^4-10^5 rows); up to 4096 rows they stay in LDS and
+ * registers, above that work vectors take 9 n doubles per resident
  * workgroup. */
 int cm_batch_solve(int nitems, const cm_system *systems, const double *const *B, double *const *X,
                    const double *tol, const int *NMAX, int restart_true, double *resval, int *iter, int *info);
@@ -196,7 +198,9 @@ int cm_system_block_time_spmm(cm_system sys, char which, int bits, int reps, dou
  * precision, times each available SpMV format (see cm_system_spmv_format)
  * and keeps the fastest.  tiles[6]: the tile choices, 0 for an absent
  * matrix.  Results of later solves are unchanged up to the summation order
- * of the row sums and of the row blocks' partial dot products. */
+ * of the row sums and of the row blocks' partial dot products.  Later
+ * single-RHS solves (apply mode E, at most 524288 rows) run in one launch
+ * where the matrices suit it. */
 int cm_system_autotune(cm_system sys, int reps, int *tiles);
 /* SpMV format of one resident matrix copy: bits 64, 32 or 16 (after
  * cm_system_enable_mixed), which 0..5 = A, G, H, G^T, L, U, format
