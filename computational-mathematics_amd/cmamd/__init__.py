@@ -143,11 +143,13 @@ def _type_host(lib):
 
 
 def _take(lib, p, count, dtype):
-    """A numpy array over a new[]-allocated one, released with its last view."""
+    """A numpy array over a new[]-allocated one, released with its last view
+    (at the interpreter's end only if there is none: exit handlers, daemon
+    threads and __del__ methods may still read it)."""
     if not p:
         return None
     buf = ((C.c_double if dtype == np.float64 else C.c_int) * max(count, 1)).from_address(p)
-    weakref.finalize(buf, lib.cm_free_d if dtype == np.float64 else lib.cm_free_i, p)
+    weakref.finalize(buf, lib.cm_free_d if dtype == np.float64 else lib.cm_free_i, p).atexit = False
     return np.frombuffer(buf, dtype=dtype)[:count]
 
 
