@@ -299,7 +299,7 @@ SOLVE_SYMBOLS = [
     "cm_system_kernel_format_bytes",
     "cm_system_enable_mixed", "cm_system_solve_mixed",
     "cm_system_block_set", "cm_system_block_get", "cm_system_block_solve", "cm_system_block_solve_mixed",
-    "cm_system_graphs", "cm_system_block_graphs", "cm_system_block_release",
+    "cm_system_graphs", "cm_system_resident", "cm_system_block_graphs", "cm_system_block_release",
     "cm_system_block_time_spmm", "cm_system_dia_info", "cm_batch_solve", "cm_system_autotune", "cm_system_block_autotune",
     "cm_system_spmv_format", "cm_system_spmv_formats", "cm_system_profile_sampled", "cm_system_block_dia", "cm_last_error", "cm_device_count",
     "cm_server_create", "cm_server_configure", "cm_server_destroy", "cm_server_add_system", "cm_server_submit", "cm_server_wait",
@@ -344,6 +344,8 @@ def _type_solve(lib):
     lib.cm_system_block_graphs.argtypes = [vp, C.c_int]
     lib.cm_system_graphs.argtypes = [vp, C.c_int]
     lib.cm_system_graphs.restype = C.c_int
+    lib.cm_system_resident.argtypes = [vp, C.c_int, C.c_int, C.c_int, C.POINTER(C.c_longlong)]
+    lib.cm_system_resident.restype = C.c_int
     lib.cm_system_block_release.argtypes = [vp]
     lib.cm_system_dia_info.argtypes = [vp, C.c_int, C.POINTER(C.c_int), C.POINTER(C.c_int),
                                        C.POINTER(C.c_longlong)]
@@ -512,6 +514,14 @@ class System:
     def graphs(self, on=True):
         """Single-RHS passes from captured hipGraphs (on) or kernel by kernel."""
         _check(self._lib.cm_system_graphs(self._h, 1 if on else 0))
+
+    def resident(self, on=True, spins=-1, join_us=-1):
+        """Solves in one launch on or off, and the limits of their waits (-1:
+        the defaults); returns the right-hand sides (solved so, not arrived,
+        given up) so far."""
+        c = (C.c_longlong * 3)()
+        _check(self._lib.cm_system_resident(self._h, int(on), int(spins), int(join_us), c))
+        return tuple(c)
 
     def block_dia(self, on=True):
         """Block products in the diagonal format where a matrix suits it (default on)."""

@@ -1217,6 +1217,19 @@ struct RsPlan {
     int count = 0;
 };
 
+// A system's resident solves: whether they are taken, how long their waits
+// last, and what became of them (columns).  One per system, which its solvers
+// of all precisions and widths share.
+struct RsControl {
+    bool on = true;
+    int spins = RS_SPINS;
+    long long join_ticks = RS_JOIN_TICKS;
+    long long solved = 0;  // columns solved in resident launches
+    long long absent = 0;  // columns whose grid did not arrive
+    long long given_up = 0;  // columns in which a wait gave up
+    int skip = 0;  // solves that are not to try
+};
+
 // What a solver keeps for its resident solves (cm_resident.hpp), made on
 // first use: reduction slots and control words on the device, the columns'
 // results in pinned memory.
@@ -1226,7 +1239,8 @@ struct RsRunner {
     RsCtl *ctl = nullptr;
     RsTable<T, VA, VF> *args = nullptr;
     SolveState *out = nullptr;
-    int slot_cols = 0, skip = 0;
+    int slot_cols = 0;
+    std::shared_ptr<RsControl> control;
     ~RsRunner()
     {
         (void)hipFree(slots);
@@ -1353,7 +1367,8 @@ struct RsRunner {
         return CM_OK;
     }
     // Runs the columns of a (its matrices and buffers filled in here).  ran:
-    // all of them did; else x is as it was in those that did not.
+    // all of them did; else x is as it was in those that did not (a.save; on a
+    // zero start it need not be).
     int run(RsArgs<T, VA, VF> &a, const DevCsr<VA> &A, const DevCsr<VF> &H, const DevCsr<VF> &G, const RsPlan &p,
             hipStream_t stream, bool &ran)
     {
@@ -1363,8 +1378,8 @@ struct RsRunner {
         const int cap = cus(&dev);
         CM_TRY(ensure(nc));
         std::memset(out, 0, RS_COLS * sizeof(SolveState));
-        if (skip > 0) {
-            skip--;
+        if (control->skip > 0) {
+            control->skip--;
             return CM_OK;
         }
         for (int q = 0; q < p.count; q++) wgs[q] = p.s[q].wgs * nc;
@@ -1382,6 +1397,8 @@ struct RsRunner {
         a.slots = slots;
         a.ctl = ctl;
         a.out = out;
+        a.spins = control->spins;
+        a.join_ticks = control->join_ticks;
         const dim3 grid(s.wgs, nc);
         k_rs_prep<T, VA, VF><<<vec_grid(a.n), BS, 0, stream>>>(a, args);
         if (s.bsz == 256) k_rs_solve<T, VA, VF, 256, 1><<<grid, 256, 0, stream>>>(args);
@@ -1391,9 +1408,24 @@ struct RsRunner {
         CM_HIP(hipGetLastError());
         CM_HIP(hipStreamSynchronize(stream));
         ran = true;
-        for (int c = 0; c < nc; c++) ran = ran && out[c].done;
+        for (int c = 0; c < nc; c++) {
+            if (out[c].done) {
+                control->solved++;
+                continue;
+            }
+            ran = false;
+            if (!a.zero_start)
+                k_rs_restore<T><<<vec_grid(a.n), BS, 0, stream>>>(a.n, a.stride, a.col[c], a.save, a.x);
+        }
+        if (ran) return CM_OK;
+        CM_HIP(hipGetLastError());
+        RsCtl h;  // did the grid arrive?
+        CM_HIP(hipMemcpyAsync(&h, ctl, sizeof h, hipMemcpyDeviceToHost, stream));
+        CM_HIP(hipStreamSynchronize(stream));
+        for (int c = 0; c < nc; c++)
+            if (!out[c].done) (h.verdict == 1 ? control->given_up : control->absent)++;
         // a device too busy for the grid: the next solves do not try
-        if (!ran) skip = RS_SKIP;
+        control->skip = RS_SKIP;
         return CM_OK;
     }
 };
@@ -1795,7 +1827,7 @@ struct Krylov {
     int run_resident(double tol, int NMAX, int info_in, int trace_cap, bool zero_start, SolveState &fin, bool &ran)
     {
         ran = false;
-        if (!resident || prof.on || (variant == 2 && mode != 'E')) return CM_OK;
+        if (!resident || !rs.control->on || prof.on || (variant == 2 && mode != 'E')) return CM_OK;
         RsPlan plan;
         CM_TRY(rs.plan(n, 1, true, A, sym ? GT : H, G, stream, plan));
         if (plan.count == 0) return CM_OK;
@@ -1817,6 +1849,7 @@ struct Krylov {
         a.idv = idv;
         a.b = b;
         a.x = x;
+        a.save = v;
         T *ex[6] = {p, tm, pc, s, t1, sc};
         for (int q = 0; q < 6; q++) a.ex[q] = ex[q];
         CM_TRY(rs.run(a, A, sym ? GT : H, G, plan, stream, ran));
@@ -1986,6 +2019,7 @@ static int create_k64(K64 &k, const HostSys &h, hipStream_t strm)
 template <class KI>
 static int create_inner(KI &ki, K64 &k)
 {
+    ki.rs.control = k.rs.control;
     // 16-bit indices for the low-precision products (built once, shared)
     for (DevCsr<double> *m : {&k.A, &k.G, &k.H, &k.GT, &k.L, &k.U})
         if (m->present() && !m->d16) CM_TRY(build_idx16(*m, k.stream));
@@ -2338,6 +2372,7 @@ struct BlockKrylov {
         G = &k.G;
         Hm = k.sym ? &k.GT : &k.H;
         idv = k.idv;
+        rs.control = k.rs.control;
         CM_TRY(make_bins(bA, *A, stream));
         CM_TRY(make_bins(bG, *G, stream));
         CM_TRY(make_bins(bH, *Hm, stream));
@@ -2612,7 +2647,7 @@ struct BlockKrylov {
         const int nc = (int)cols.size();
         RsPlan plan;
         int per = nc;
-        if (nc == 0) return CM_OK;
+        if (nc == 0 || !rs.control->on) return CM_OK;
         CM_TRY(rs.plan(n, per, false, *A, *Hm, *G, stream, plan));
         if (plan.count == 0 && sizeof(T) == 4 && nc > 1) {
             per = (nc + 1) / 2;
@@ -2637,6 +2672,7 @@ struct BlockKrylov {
             a.idv = idv;
             a.b = b;
             a.x = x;
+            a.save = v;
             T *ex[6] = {p, tm, pc, s, t, sc};
             for (int q = 0; q < 6; q++) a.ex[q] = ex[q];
             bool ok;
@@ -3179,6 +3215,7 @@ static int system_create(System &S, const HostSys &h)
     S.variant = h.variant;
     CM_HIP(hipStreamCreateWithFlags(&S.stream, hipStreamNonBlocking));
     S.k64 = std::make_unique<K64>();
+    S.k64->rs.control = std::make_shared<RsControl>();
     return create_k64(*S.k64, h, S.stream);
 }
 
@@ -3718,6 +3755,22 @@ int cm_system_graphs(cm_system h, int on)
     if (S.k32) S.k32->use_graph = on != 0;
     if (S.k16) S.k16->use_graph = on != 0;
     S.graphs = on != 0;
+    return CM_OK;
+}
+
+int cm_system_resident(cm_system h, int on, int spins, int join_us, long long *counts)
+{
+    if (!h) return fail(CM_ERR_ARG, "null handle");
+    RsControl &c = *h->sys.k64->rs.control;
+    c.on = on != 0;
+    c.skip = 0;
+    c.spins = spins < 0 ? RS_SPINS : std::min(spins, RS_SPINS);
+    c.join_ticks = join_us < 0 ? RS_JOIN_TICKS : std::min(100LL * join_us, RS_JOIN_TICKS);
+    if (counts) {
+        counts[0] = c.solved;
+        counts[1] = c.absent;
+        counts[2] = c.given_up;
+    }
     return CM_OK;
 }
 

@@ -42,7 +42,12 @@
 // have arrived: each counts itself in, the first closes the count when the
 // grid is complete or after RS_JOIN_TICKS, and if anyone is missing then all
 // leave and the caller takes the launch-per-operation path.  All other waits
-// end after RS_SPINS loads, with the same result.
+// end after RS_SPINS loads.  A workgroup whose wait ended so leaves without
+// writing its rows of x, and a column counts as solved only when all its
+// workgroups have written theirs: others may still get through the reduction
+// that one gave up on, if its own sums were out by then.  The host gives the
+// columns that do not count their starting x back (k_rs_restore) and takes
+// the launch-per-operation path for them.
 #pragma once
 #include "cm_kernels.hpp"
 
@@ -130,12 +135,15 @@ __device__ __forceinline__ X *rs_glob(X *p)
     return (X *)(__attribute__((address_space(1))) X *)p;
 }
 
+constexpr int RS_COLS = 16;  // columns of a launch at most
+
 // Control words of one launch, cleared by k_rs_prep.
 struct RsCtl {
     unsigned join;  // arrivals; top bit: closed
     unsigned pad0[31];
     unsigned verdict;  // 1: all arrived, 2: leave
     unsigned pad1[31];
+    unsigned fin[RS_COLS];  // workgroups of a column that wrote their x
 };
 
 // One matrix of the solve: diagonals with a CSR remainder (nd diagonals), or
@@ -180,17 +188,17 @@ static bool rs_windows(const std::vector<int> &off, int bsz, int rows, RsMat<V> 
 
 // Column k of the launch (blockIdx.y) is column col[k] of b and x, which hold
 // `stride` columns interleaved, and solves to tol[k].
-constexpr int RS_COLS = 16;
 template <class T, class VA, class VF>
 struct RsArgs {
-    int n, nmax, variant, maxmsteps, info_in, zero_start, trace_cap, stride, ncols;
+    int n, nmax, variant, maxmsteps, info_in, zero_start, trace_cap, stride, ncols, spins;
+    long long join_ticks;
     int col[RS_COLS];
     double tol[RS_COLS], eps;
     double *trace;  // device; first column
     RsMat<VF> H, G;
     RsMat<VA> A;
     const T *idv, *b;
-    T *x;
+    T *x, *save;      // save: the starting x (n x stride), not used on a zero start
     T *ex[6];         // exchanged vectors of ncols x n: p, H p, M p, s, H s, M s
     double *slots;    // ncols x RS_SETS x RS_K x RS_WGS
     RsCtl *ctl;
@@ -227,8 +235,8 @@ __global__ __launch_bounds__(RS_GROUP) void k_row_spread(int n, const int *ptr, 
     if (threadIdx.x == 0) atomicMax(out + 1, ptr[min(r0 + RS_GROUP, n)] - ptr[r0]);
 }
 
-// Markers into the exchanged vectors and reduction slots, control words 0,
-// and the arguments to where the solve reads them (every column's pointers
+// Markers into the exchanged vectors and reduction slots, control words 0, the
+// starting x kept, and the arguments to where the solve reads them (every column's pointers
 // ready: computed in the solve they made a pass 1.5% slower).
 template <class T, class VA, class VF>
 __global__ __launch_bounds__(BS) void k_rs_prep(RsArgs<T, VA, VF> a, RsTable<T, VA, VF> *to)
@@ -241,11 +249,14 @@ __global__ __launch_bounds__(BS) void k_rs_prep(RsArgs<T, VA, VF> a, RsTable<T, 
     }
     for (int i = t0; i < a.ncols * RS_SETS * RS_K * RS_WGS; i += st)
         reinterpret_cast<unsigned long long *>(a.slots)[i] = RsBits<double>::MARK;
+    if (!a.zero_start)
+        for (int i = t0; i < a.n * a.stride; i += st) a.save[i] = a.x[i];
     if (t0 == 0) {
         a.ctl->join = 0;
         a.ctl->verdict = 0;
         to->a = a;
     }
+    if (t0 < RS_COLS) a.ctl->fin[t0] = 0;
     if (t0 < a.ncols) {
         RsCol<T> c;
         int col = 0;
@@ -266,8 +277,18 @@ __global__ __launch_bounds__(BS) void k_rs_prep(RsArgs<T, VA, VF> a, RsTable<T, 
     }
 }
 
+// Column col of x as it was before the launch.
+template <class T>
+__global__ __launch_bounds__(BS) void k_rs_restore(int n, int stride, int col, const T *__restrict__ save,
+                                                   T *__restrict__ x)
+{
+    for (int i = blockIdx.x * BS + threadIdx.x; i < n; i += gridDim.x * BS)
+        x[(size_t)i * stride + col] = save[(size_t)i * stride + col];
+}
+
 // x[j[q]] for the q with j[q] >= 0 (0 otherwise), waiting for entries that
-// are not there yet; *dead is set (and honoured) when a wait gives up.
+// are not there yet; dead[0] is set (and honoured) when a wait gives up, after
+// dead[1] loads.
 template <class T, int R>
 __device__ __forceinline__ void rs_gather(const T *x, const int (&j)[R], T (&v)[R], volatile int *dead)
 {
@@ -280,7 +301,7 @@ __device__ __forceinline__ void rs_gather(const T *x, const int (&j)[R], T (&v)[
 #pragma unroll
         for (int q = 0; q < R; q++) miss |= b[q] == B::MARK;
         if (!miss) break;
-        if (++spin >= RS_SPINS) *dead = 1;
+        if (++spin >= dead[1]) *dead = 1;
         if (*dead) break;
 #pragma unroll
         for (int q = 0; q < R; q++)
@@ -555,7 +576,7 @@ __device__ __forceinline__ void rs_allsum(double (&v)[RS_K], double *slots, int 
     double *base = slots + (size_t)set * K * RS_WGS;
     if (w == 0) {
         const double q = rs_group_sum<NW>(lane < K * NW ? red[lane] : 0.0);
-        // a workgroup that gave up withholds its sums, so nobody finishes without it
+        // a workgroup that gave up withholds its sums, so nobody goes on without it
         if (lane < K * NW && lane % NW == 0 && !*dead) rs_put(base + (lane / NW) * RS_WGS + blockIdx.x, q);
     }
     if (w < C) {  // wave w adds workgroups [w * WAVE, (w + 1) * WAVE)
@@ -580,7 +601,7 @@ __device__ __forceinline__ void rs_allsum(double (&v)[RS_K], double *slots, int 
 }
 
 // Arrival of the grid; true when every workgroup is running.
-__device__ __forceinline__ bool rs_join(RsCtl *c, int *sh)
+__device__ __forceinline__ bool rs_join(RsCtl *c, long long ticks, int *sh)
 {
     const unsigned all = gridDim.x * gridDim.y;
     if (threadIdx.x == 0) {
@@ -591,7 +612,7 @@ __device__ __forceinline__ bool rs_join(RsCtl *c, int *sh)
             if (q == 0) {
                 const long long t0 = wall_clock64();
                 while (__hip_atomic_load(&c->join, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) < all &&
-                       wall_clock64() - t0 < RS_JOIN_TICKS) {
+                       wall_clock64() - t0 < ticks) {
                 }
                 const unsigned f = __hip_atomic_fetch_or(&c->join, CLOSED, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
                 verdict = f == all ? 1u : 2u;
@@ -612,12 +633,13 @@ __device__ __forceinline__ bool rs_join(RsCtl *c, int *sh)
 
 // The reference loop (AFIIM/src/bicgstab.cpp:149-281, ACIFIM's non-finite
 // alpha guard, ACIFIM/src/bicgstab.cpp:208-213) on R rows per thread: row
-// (blockIdx * R + q) * BSZ + thread.  out->done is set when the solve ran;
-// when it did not (the grid did not arrive, or a wait gave up), x is as it
-// was.  One loop iteration is half a pass: step 2 applies M and A to p and ends
-// in alpha, step 5 to s and ends in omega; step 6 is the initial residual.  The new r0 . r is formed from the sums the omega
-// reduction carries anyway, r0 . s - omega (r0 . t), where r0 . s is what
-// rounding leaves of 0; this saves an exchange of 2 us per pass.
+// (blockIdx * R + q) * BSZ + thread.  out->done is set when all workgroups of
+// the column wrote their x; when the grid did not arrive x is as it was, when
+// a wait gave up some rows may be written.  One loop iteration is half a pass:
+// step 2 applies M and A to p and ends in alpha, step 5 to s and ends in
+// omega; step 6 is the initial residual.  The new r0 . r is formed from the
+// sums the omega reduction carries anyway, r0 . s - omega (r0 . t), where
+// r0 . s is what rounding leaves of 0; this saves an exchange of 2 us per pass.
 template <class T, class VA, class VF, int BSZ, int R>
 __global__ __launch_bounds__(BSZ) void k_rs_solve(const RsTable<T, VA, VF> *args)
 {
@@ -627,10 +649,13 @@ __global__ __launch_bounds__(BSZ) void k_rs_solve(const RsTable<T, VA, VF> *args
     __shared__ Acc prod[RS_PER * BSZ];
     __shared__ T win[rs_steps(BSZ) * BSZ];
     __shared__ double red[RS_SETS][RS_K * (BSZ / WAVE + RS_WGS / WAVE)];
-    __shared__ int sh_join, sh_dead;
-    if (threadIdx.x == 0) sh_dead = 0;
-    if (!rs_join(g->ctl, &sh_join)) return;
-    volatile int *dead = &sh_dead;
+    __shared__ int sh_join, sh_dead[2];  // a wait gave up; loads until one does
+    if (threadIdx.x == 0) {
+        sh_dead[0] = 0;
+        sh_dead[1] = g->spins;
+    }
+    if (!rs_join(g->ctl, g->join_ticks, &sh_join)) return;
+    volatile int *dead = sh_dead;
     const int n = g->n, tid = threadIdx.x;
     int row0 = (int)blockIdx.x * R * BSZ;
     T x[R], r[R], r0[R], p[R], v[R], w[R], dv[R];  // w: M p, then M s
@@ -839,14 +864,19 @@ __global__ __launch_bounds__(BSZ) void k_rs_solve(const RsTable<T, VA, VF> *args
         const int i = row0 + q * BSZ + tid;
         if (i < n && (g->nmax > 0 || g->zero_start)) rs_glob(c->x)[(size_t)i * g->stride] = x[q];
     }
-    if (blockIdx.x == 0 && tid == 0) {
+    if (tid == 0) {
         SolveState *o = c->out;
-        o->ro = ro;
-        o->rc = rc;
-        o->iter = iter;
-        o->info = info;
-        o->ntrace = ntrace;
-        o->done = 1;
+        if (blockIdx.x == 0) {
+            o->ro = ro;
+            o->rc = rc;
+            o->iter = iter;
+            o->info = info;
+            o->ntrace = ntrace;
+        }
+        // after the last reduction a workgroup's waves all come here or none
+        // does; what they wrote is in place when the launch has ended
+        const unsigned q = __hip_atomic_fetch_add(&g->ctl->fin[blockIdx.y], 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        if (q + 1 == gridDim.x) o->done = 1;
     }
 }
 

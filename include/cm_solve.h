@@ -148,6 +148,15 @@ int cm_system_block_get(cm_system sys, double *X);
  * (tuned systems and blocks of at most 524288 rows) do so in both cases. */
 int cm_system_graphs(cm_system sys, int on);
 int cm_system_block_graphs(cm_system sys, int on);
+/* Solves in one launch (resident solves) of this system: taken where they
+ * suit it (on, the default) or never (off: launched passes).  spins and
+ * join_us lower the looks of one wait and the time a grid has to arrive
+ * before the launched passes run instead, for tests of that (-1: the
+ * default limits).  counts (or null) receives the right-hand sides so far
+ * that resident launches solved, whose grid did not arrive, and in which a
+ * wait was given up: the latter two took the launched passes from their
+ * starting x. */
+int cm_system_resident(cm_system sys, int on, int spins, int join_us, long long counts[3]);
 /* Persistent batched solves: nitems right-hand sides of small resident
  * systems (item i: system systems[i], column B[i], initial guess and result
  * X[i], tol[i], NMAX[i]; systems may repeat and differ in size) in one
