@@ -25,6 +25,7 @@
 //    low-precision matrices are cast on the device from the resident FP64
 //    ones and share their index arrays.
 #include <hip/hip_runtime.h>
+#include <unistd.h>
 
 #include <algorithm>
 #include <chrono>
@@ -1163,7 +1164,9 @@ struct HostSys {
 // CUs promised to resident grids, per device: a grid waits for all its
 // workgroups, so grids whose workgroups together exceed the CUs are not in
 // flight at once (from several threads, or a server's workers).  Each
-// workgroup counts as a CU.
+// workgroup counts as a CU.  Grids take their turns in the order they came: a
+// solve is not done another way because the device is busy, which would make
+// its last bits depend on what else runs.
 class ResidentGate {
   public:
     static ResidentGate &get()
@@ -1172,49 +1175,47 @@ class ResidentGate {
         return g;
     }
     static constexpr int MAX_DEV = 64;
-    // The first of the nc sizes wgs[] that fits the CUs not promised, waiting
-    // up to WAIT for one to fit; its index, or -1 (the caller's launched
-    // passes need no promise).
-    static constexpr std::chrono::milliseconds WAIT{3};
-    int acquire(int dev, const int *wgs, int nc, int cus)
+    // Waits until wgs <= cap workgroups and those promised fit cap.
+    void acquire(int dev, int wgs, int cap)
     {
-        if (dev < 0 || dev >= MAX_DEV) return -1;
-        int got = -1;
-        auto fits = [&] {
-            for (got = 0; got < nc; got++)
-                if (used[dev] + wgs[got] <= cus) return true;
-            got = -1;
-            return false;
-        };
+        Dev &d = at(dev);
         std::unique_lock<std::mutex> lk(mu);
-        if (!cv.wait_for(lk, WAIT, fits)) return -1;
-        used[dev] += wgs[got];
-        return got;
+        const long long me = d.next++;
+        cv.wait(lk, [&] { return me == d.turn && d.used + wgs <= cap; });
+        d.turn++;
+        d.used += wgs;
+        lk.unlock();
+        cv.notify_all();  // the next one may fit too
     }
     void release(int dev, int wgs)
     {
         {
             std::lock_guard<std::mutex> lk(mu);
-            used[dev] -= wgs;
+            at(dev).used -= wgs;
         }
         cv.notify_all();
     }
 
   private:
+    struct Dev {
+        int used = 0;
+        long long next = 0, turn = 0;
+    };
+    Dev &at(int dev) { return devs[dev % MAX_DEV]; }
     std::mutex mu;
     std::condition_variable cv;
-    int used[MAX_DEV] = {};
+    Dev devs[MAX_DEV];
 };
 
-// A launch shape of a resident solve (threads and rows per thread of its
-// workgroups, and the workgroups of one column), and the shapes a solve can
-// take, the preferred one first.
+// The launch shape of a resident solve (threads and rows per thread of its
+// workgroups, and the workgroups of one column), and the columns one launch
+// takes at most (0: none suits).
 struct RsShape {
     int bsz, rows, wgs;
 };
 struct RsPlan {
-    RsShape s[4];
-    int count = 0;
+    RsShape s{0, 0, 0};
+    int per = 0;
 };
 
 // A system's resident solves: whether they are taken, how long their waits
@@ -1316,32 +1317,37 @@ struct RsRunner {
         if (!out) CM_HIP(hipHostMalloc((void **)&out, RS_COLS * sizeof(SolveState), hipHostMallocDefault));
         return CM_OK;
     }
-    // The shapes whose grids for nc columns fit the device, one workgroup per
-    // CU.  Small workgroups run a pass faster (46656 rows, FP64: 28 us on 512
-    // rows, 37 on 1024 and 58 on 2048; FP32: 30, 31 and 38), large ones leave
-    // CUs to other solves: smallest first for a lone column (`all`) and in
-    // FP64; a block in FP32 first the smallest that takes at most half of the
-    // CUs, else the largest (a burst of 24 requests on six systems took 9 ms
-    // instead of 13 with the smallest first, where the grids had to wait for
-    // each other).
+    // The shape of an n-row solve: a lone right-hand side (width 0) or a block
+    // of the given width, one workgroup per CU.  It depends on the system and
+    // the width alone, not on the columns still active or the CUs free, so a
+    // column's sums are formed the same way every time.  Small workgroups run
+    // a pass faster (46656 rows, FP64: 28 us on 512 rows, 37 on 1024 and 58 on
+    // 2048; FP32: 30, 31 and 38), large ones leave CUs to other solves: the
+    // smallest that fits for a lone column and in FP64; a block in FP32 the
+    // smallest that takes at most half of the CUs, else the largest (a burst
+    // of 24 requests on six systems took 9 ms instead of 13 with the smallest,
+    // where the grids had to wait for each other), and if that does not fit
+    // either, the largest in two launches (FP64 halves took longer than the
+    // launched passes).
     // Entries in CSR are gathered past the L2s, RS_PER * bsz at a time, and
     // added by their row's thread.  Launched / resident us per pass of FP64,
     // by these gather steps of the three products: 62 / 40 at 256^2 rows on
     // 1.8 steps, 102 / 73 at 512^2 on 3.7, 73 / 72 at 64^3 on 7, 158 / 154 at
     // 724^2 on 7.4 (FP32 112 / 85); 90 / 2160 at 90^2 rows of 370 entries, on
     // 53 steps whose long rows are summed serially.
-    int plan(int n, int nc, bool all, const DevCsr<VA> &A, const DevCsr<VF> &H, const DevCsr<VF> &G,
-             hipStream_t stream, RsPlan &p)
+    int plan(int n, int width, const DevCsr<VA> &A, const DevCsr<VF> &H, const DevCsr<VF> &G, hipStream_t stream,
+             RsPlan &p)
     {
-        p.count = 0;
-        if (n < 1 || n > RS_MAX_ROWS || nc > RS_COLS) return CM_OK;
+        p.per = 0;
+        if (n < 1 || n > RS_MAX_ROWS || width > RS_COLS) return CM_OK;
         int dev = 0;
-        const int cap = cus(&dev);
+        const int cap = cus(&dev), cols = std::max(width, 1);
         for (const RsShape &s : {RsShape{256, 1, 0}, RsShape{512, 1, 0}, RsShape{512, 2, 0}, RsShape{512, 4, 0}}) {
             const int rows = s.bsz * s.rows;
             RsShape f = s;
             f.wgs = (n + rows - 1) / rows;
-            if ((long long)f.wgs * nc > cap) continue;
+            const int per = std::min(cols, cap / f.wgs);
+            if (per < cols && (sizeof(T) == 8 || 2 * per < cols)) continue;
             RowSpread w[3];
             CM_TRY(spread(A, s.bsz, rows, stream, w[0]));
             CM_TRY(spread(H, s.bsz, rows, stream, w[1]));
@@ -1352,29 +1358,23 @@ struct RsRunner {
                 serial += q.longest;
             }
             if (steps > RS_CSR_STEPS * (1.0 + (double)n / RS_MAX_ROWS) || serial > RS_CSR_ROW) continue;
-            p.s[p.count++] = f;
-            if (all) return CM_OK;
+            p.s = f;
+            p.per = per;
+            if (width == 0 || sizeof(T) == 8 || 2 * f.wgs * cols <= cap) break;
         }
-        if (p.count == 0 || sizeof(T) == 8) return CM_OK;
-        int first = 0;
-        while (first < p.count && p.s[first].wgs * nc > cap / 2) first++;
-        if (first == p.count) {  // every shape takes more than half
-            std::reverse(p.s, p.s + p.count);
-            return CM_OK;
-        }
-        p.count -= first;
-        for (int q = 0; q < p.count; q++) p.s[q] = p.s[q + first];
         return CM_OK;
     }
     // Runs the columns of a (its matrices and buffers filled in here).  ran:
     // all of them did; else x is as it was in those that did not (a.save; on a
     // zero start it need not be).
+    // A grid that does not arrive in RS_JOIN_TICKS leaves and is tried again,
+    // RS_TRIES times with pauses: by then kernels of some 0.3 s have ended.
     int run(RsArgs<T, VA, VF> &a, const DevCsr<VA> &A, const DevCsr<VF> &H, const DevCsr<VF> &G, const RsPlan &p,
             hipStream_t stream, bool &ran)
     {
         ran = false;
         const int nc = a.ncols;
-        int dev = 0, wgs[4];
+        int dev = 0;
         const int cap = cus(&dev);
         CM_TRY(ensure(nc));
         std::memset(out, 0, RS_COLS * sizeof(SolveState));
@@ -1382,15 +1382,14 @@ struct RsRunner {
             control->skip--;
             return CM_OK;
         }
-        for (int q = 0; q < p.count; q++) wgs[q] = p.s[q].wgs * nc;
-        const int pick = ResidentGate::get().acquire(dev, wgs, p.count, cap);
-        if (pick < 0) return CM_OK;
+        const RsShape &s = p.s;
+        const int rows = s.bsz * s.rows;
+        if (s.wgs * nc > cap) return CM_OK;  // another device than planned for
         struct Held {
             int dev, wgs;
+            Held(int d, int w, int cap) : dev(d), wgs(w) { ResidentGate::get().acquire(dev, wgs, cap); }
             ~Held() { ResidentGate::get().release(dev, wgs); }
-        } held{dev, wgs[pick]};
-        const RsShape &s = p.s[pick];
-        const int rows = s.bsz * s.rows;
+        } held(dev, s.wgs * nc, cap);
         a.A = mat(A, s.bsz, rows);
         a.H = mat(H, s.bsz, rows);
         a.G = mat(G, s.bsz, rows);
@@ -1400,32 +1399,40 @@ struct RsRunner {
         a.spins = control->spins;
         a.join_ticks = control->join_ticks;
         const dim3 grid(s.wgs, nc);
-        k_rs_prep<T, VA, VF><<<vec_grid(a.n), BS, 0, stream>>>(a, args);
-        if (s.bsz == 256) k_rs_solve<T, VA, VF, 256, 1><<<grid, 256, 0, stream>>>(args);
-        else if (s.rows == 1) k_rs_solve<T, VA, VF, 512, 1><<<grid, 512, 0, stream>>>(args);
-        else if (s.rows == 2) k_rs_solve<T, VA, VF, 512, 2><<<grid, 512, 0, stream>>>(args);
-        else k_rs_solve<T, VA, VF, 512, 4><<<grid, 512, 0, stream>>>(args);
-        CM_HIP(hipGetLastError());
-        CM_HIP(hipStreamSynchronize(stream));
-        ran = true;
-        for (int c = 0; c < nc; c++) {
-            if (out[c].done) {
-                control->solved++;
-                continue;
+        for (int attempt = 1;; attempt++) {
+            k_rs_prep<T, VA, VF><<<vec_grid(a.n), BS, 0, stream>>>(a, args);
+            if (s.bsz == 256) k_rs_solve<T, VA, VF, 256, 1><<<grid, 256, 0, stream>>>(args);
+            else if (s.rows == 1) k_rs_solve<T, VA, VF, 512, 1><<<grid, 512, 0, stream>>>(args);
+            else if (s.rows == 2) k_rs_solve<T, VA, VF, 512, 2><<<grid, 512, 0, stream>>>(args);
+            else k_rs_solve<T, VA, VF, 512, 4><<<grid, 512, 0, stream>>>(args);
+            CM_HIP(hipGetLastError());
+            CM_HIP(hipStreamSynchronize(stream));
+            int done = 0;
+            for (int c = 0; c < nc; c++) done += out[c].done;
+            control->solved += done;
+            if (done == nc) {
+                ran = true;
+                return CM_OK;
             }
-            ran = false;
-            if (!a.zero_start)
-                k_rs_restore<T><<<vec_grid(a.n), BS, 0, stream>>>(a.n, a.stride, a.col[c], a.save, a.x);
+            RsCtl h;  // did the grid arrive?
+            CM_HIP(hipMemcpyAsync(&h, ctl, sizeof h, hipMemcpyDeviceToHost, stream));
+            CM_HIP(hipStreamSynchronize(stream));
+            if (h.verdict == 1) {
+                control->given_up += nc - done;
+                for (int c = 0; c < nc && !a.zero_start; c++)
+                    if (!out[c].done)
+                        k_rs_restore<T><<<vec_grid(a.n), BS, 0, stream>>>(a.n, a.stride, a.col[c], a.save, a.x);
+                CM_HIP(hipGetLastError());
+                break;
+            }
+            if (attempt == RS_TRIES) {
+                control->absent += nc;
+                break;
+            }
+            // not all threads and processes at the same moments
+            std::this_thread::sleep_for(std::chrono::microseconds(500 * attempt + 37 * (dev + getpid() % 64)));
         }
-        if (ran) return CM_OK;
-        CM_HIP(hipGetLastError());
-        RsCtl h;  // did the grid arrive?
-        CM_HIP(hipMemcpyAsync(&h, ctl, sizeof h, hipMemcpyDeviceToHost, stream));
-        CM_HIP(hipStreamSynchronize(stream));
-        for (int c = 0; c < nc; c++)
-            if (!out[c].done) (h.verdict == 1 ? control->given_up : control->absent)++;
-        // a device too busy for the grid: the next solves do not try
-        control->skip = RS_SKIP;
+        control->skip = RS_SKIP;  // a device too busy for the grid: the next solves do not try
         return CM_OK;
     }
 };
@@ -1829,8 +1836,8 @@ struct Krylov {
         ran = false;
         if (!resident || !rs.control->on || prof.on || (variant == 2 && mode != 'E')) return CM_OK;
         RsPlan plan;
-        CM_TRY(rs.plan(n, 1, true, A, sym ? GT : H, G, stream, plan));
-        if (plan.count == 0) return CM_OK;
+        CM_TRY(rs.plan(n, 0, A, sym ? GT : H, G, stream, plan));
+        if (plan.per == 0) return CM_OK;
         CM_TRY(ensure_trace(trace_cap));
         RsArgs<T, VA, VF> a;
         std::memset(&a, 0, sizeof a);
@@ -2629,11 +2636,10 @@ struct BlockKrylov {
     }
 
     // The active columns in resident launches, each column on workgroups of
-    // its own with its own scalars and exit: all columns at once where their
-    // workgroups fit the CUs, in FP32 else in two halves (FP64 halves took
-    // longer than the launched passes).  A launched pass is some 16 kernels
-    // whatever the width.  Per pass, launched / here: 46656 rows, FP32 63 / 31
-    // us for 2 columns, 91 / 34 for 5, 92 / 42 for 8, 106 / 77 for 14 (halves),
+    // its own with its own scalars and exit: as many columns at once as their
+    // workgroups fit the CUs.  A launched pass is some 16 kernels whatever the
+    // width.  Per pass, launched / here: 46656 rows, FP32 63 / 31 us for 2
+    // columns, 91 / 34 for 5, 92 / 42 for 8, 106 / 77 for 14 (two launches),
     // FP64 61 / 29, 88 / 45, 90 / 82; 6859 rows, FP32 64-72 / 30.  active: the
     // columns to run, on return those still to run (none when ran); fin: the
     // states of those that did.
@@ -2646,14 +2652,10 @@ struct BlockKrylov {
             if (active[j]) cols.push_back(j);
         const int nc = (int)cols.size();
         RsPlan plan;
-        int per = nc;
         if (nc == 0 || !rs.control->on) return CM_OK;
-        CM_TRY(rs.plan(n, per, false, *A, *Hm, *G, stream, plan));
-        if (plan.count == 0 && sizeof(T) == 4 && nc > 1) {
-            per = (nc + 1) / 2;
-            CM_TRY(rs.plan(n, per, false, *A, *Hm, *G, stream, plan));
-        }
-        if (plan.count == 0) return CM_OK;
+        CM_TRY(rs.plan(n, KB, *A, *Hm, *G, stream, plan));
+        if (plan.per == 0) return CM_OK;
+        const int launches = (nc + plan.per - 1) / plan.per, per = (nc + launches - 1) / launches;
         for (int c0 = 0; c0 < nc; c0 += per) {
             RsArgs<T, VA, VF> a;
             std::memset(&a, 0, sizeof a);

@@ -41,7 +41,8 @@
 // most one workgroup per CU, and a workgroup starts working only when all
 // have arrived: each counts itself in, the first closes the count when the
 // grid is complete or after RS_JOIN_TICKS, and if anyone is missing then all
-// leave and the caller takes the launch-per-operation path.  All other waits
+// leave; the caller launches the grid again and at last takes the
+// launch-per-operation path.  All other waits
 // end after RS_SPINS loads.  A workgroup whose wait ended so leaves without
 // writing its rows of x, and a column counts as solved only when all its
 // workgroups have written theirs: others may still get through the reduction
@@ -61,7 +62,8 @@ constexpr int RS_SPINS = 1 << 20;          // loads of one entry before a wait g
 constexpr int RS_GROUP = 256;              // rows over which the spread of CSR entries is taken
 constexpr double RS_CSR_STEPS = 4.0;       // gather steps of the three products' CSR entries (twice that at the most rows)
 constexpr double RS_CSR_ROW = 256.0;       // entries of the three products' longest CSR rows
-constexpr int RS_SKIP = 16;                // launched solves after a grid that did not arrive
+constexpr int RS_TRIES = 16;               // launches of a grid that does not arrive
+constexpr int RS_SKIP = 16;                // launched solves after that
 constexpr long long RS_JOIN_TICKS = 1000000;  // 100 MHz ticks the grid may take to arrive (10 ms)
 constexpr int RS_K = 4;                    // sums per reduction
 constexpr int RS_SETS = 5;                 // reduction slots: setup, alpha and omega of even and odd passes

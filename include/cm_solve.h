@@ -149,7 +149,12 @@ int cm_system_block_get(cm_system sys, double *X);
 int cm_system_graphs(cm_system sys, int on);
 int cm_system_block_graphs(cm_system sys, int on);
 /* Solves in one launch (resident solves) of this system: taken where they
- * suit it (on, the default) or never (off: launched passes).  spins and
+ * suit it (on, the default) or never (off: launched passes).  Which of the
+ * two a solve takes, and in what order it sums, depends on the system and the
+ * block width alone: grids of concurrent solves wait for their turn.  Only
+ * when other work on the device keeps a grid from starting for some 0.3 s
+ * does the solve (and the next 16) take the launched passes, whose sums
+ * differ by rounding.  spins and
  * join_us lower the looks of one wait and the time a grid has to arrive
  * before the launched passes run instead, for tests of that (-1: the
  * default limits).  counts (or null) receives the right-hand sides so far
