@@ -1175,30 +1175,35 @@ class ResidentGate {
         return g;
     }
     static constexpr int MAX_DEV = 64;
-    // Waits until wgs <= cap workgroups and those promised fit cap.
-    void acquire(int dev, int wgs, int cap)
+    // Waits until wgs <= room.grid workgroups fit with those promised: room.grid
+    // of them on CUs taken whole, room.all in all.
+    void acquire(int dev, int wgs, const RsRoom &room)
     {
         Dev &d = at(dev);
         std::unique_lock<std::mutex> lk(mu);
         const long long me = d.next++;
-        cv.wait(lk, [&] { return me == d.turn && d.used + wgs <= cap; });
+        cv.wait(lk, [&] {
+            return me == d.turn && d.used + wgs <= room.all && (!room.whole || d.whole + wgs <= room.grid);
+        });
         d.turn++;
         d.used += wgs;
+        if (room.whole) d.whole += wgs;
         lk.unlock();
         cv.notify_all();  // the next one may fit too
     }
-    void release(int dev, int wgs)
+    void release(int dev, int wgs, const RsRoom &room)
     {
         {
             std::lock_guard<std::mutex> lk(mu);
             at(dev).used -= wgs;
+            if (room.whole) at(dev).whole -= wgs;
         }
         cv.notify_all();
     }
 
   private:
     struct Dev {
-        int used = 0;
+        int used = 0, whole = 0;
         long long next = 0, turn = 0;
     };
     Dev &at(int dev) { return devs[dev % MAX_DEV]; }
@@ -1322,7 +1327,9 @@ struct RsRunner {
     // the width alone, not on the columns still active or the CUs free, so a
     // column's sums are formed the same way every time.  Small workgroups run
     // a pass faster (46656 rows, FP64: 28 us on 512 rows, 37 on 1024 and 58 on
-    // 2048; FP32: 30, 31 and 38), large ones leave CUs to other solves: the
+    // 2048; FP32: 30, 31 and 38; three rows per thread instead of four at
+    // 64^3 rows: 68 us instead of 80, and 75 launched; FP32 37, 41 and 65),
+    // large ones leave CUs to other solves: the
     // smallest that fits for a lone column and in FP64; a block in FP32 the
     // smallest that takes at most half of the CUs, else the largest (a burst
     // of 24 requests on six systems took 9 ms instead of 13 with the smallest,
@@ -1342,11 +1349,11 @@ struct RsRunner {
         if (n < 1 || n > RS_MAX_ROWS || width > RS_COLS) return CM_OK;
         int dev = 0;
         const int cap = cus(&dev), cols = std::max(width, 1);
-        for (const RsShape &s : {RsShape{256, 1, 0}, RsShape{512, 1, 0}, RsShape{512, 2, 0}, RsShape{512, 4, 0}}) {
+        for (const RsShape &s : {RsShape{256, 1, 0}, RsShape{512, 1, 0}, RsShape{512, 2, 0}, RsShape{512, 3, 0}, RsShape{512, 4, 0}}) {
             const int rows = s.bsz * s.rows;
             RsShape f = s;
             f.wgs = (n + rows - 1) / rows;
-            const int per = std::min(cols, cap / f.wgs);
+            const int room = rs_room<T>(s.bsz, s.rows, cap).grid, per = std::min(cols, room / f.wgs);
             if (per < cols && (sizeof(T) == 8 || 2 * per < cols)) continue;
             RowSpread w[3];
             CM_TRY(spread(A, s.bsz, rows, stream, w[0]));
@@ -1357,10 +1364,10 @@ struct RsRunner {
                 steps += (double)q.group * rows / RS_GROUP / (RS_PER * s.bsz);
                 serial += q.longest;
             }
-            if (steps > RS_CSR_STEPS * (1.0 + (double)n / RS_MAX_ROWS) || serial > RS_CSR_ROW) continue;
+            if (steps > RS_CSR_STEPS * (1.0 + (double)n / RS_CSR_TWICE) || serial > RS_CSR_ROW) continue;
             p.s = f;
             p.per = per;
-            if (width == 0 || sizeof(T) == 8 || 2 * f.wgs * cols <= cap) break;
+            if (width == 0 || sizeof(T) == 8 || 2 * f.wgs * cols <= room) break;
         }
         return CM_OK;
     }
@@ -1384,12 +1391,14 @@ struct RsRunner {
         }
         const RsShape &s = p.s;
         const int rows = s.bsz * s.rows;
-        if (s.wgs * nc > cap) return CM_OK;  // another device than planned for
+        const RsRoom room = rs_room<T>(s.bsz, s.rows, cap);
+        if (s.wgs * nc > room.grid) return CM_OK;  // another device than planned for
         struct Held {
-            int dev, wgs;
-            Held(int d, int w, int cap) : dev(d), wgs(w) { ResidentGate::get().acquire(dev, wgs, cap); }
-            ~Held() { ResidentGate::get().release(dev, wgs); }
-        } held(dev, s.wgs * nc, cap);
+            const int dev, wgs;
+            const RsRoom &room;
+            Held(int d, int w, const RsRoom &r) : dev(d), wgs(w), room(r) { ResidentGate::get().acquire(dev, wgs, room); }
+            ~Held() { ResidentGate::get().release(dev, wgs, room); }
+        } held(dev, s.wgs * nc, room);
         a.A = mat(A, s.bsz, rows);
         a.H = mat(H, s.bsz, rows);
         a.G = mat(G, s.bsz, rows);
@@ -1404,6 +1413,7 @@ struct RsRunner {
             if (s.bsz == 256) k_rs_solve<T, VA, VF, 256, 1><<<grid, 256, 0, stream>>>(args);
             else if (s.rows == 1) k_rs_solve<T, VA, VF, 512, 1><<<grid, 512, 0, stream>>>(args);
             else if (s.rows == 2) k_rs_solve<T, VA, VF, 512, 2><<<grid, 512, 0, stream>>>(args);
+            else if (s.rows == 3) k_rs_solve<T, VA, VF, 512, 3><<<grid, 512, 0, stream>>>(args);
             else k_rs_solve<T, VA, VF, 512, 4><<<grid, 512, 0, stream>>>(args);
             CM_HIP(hipGetLastError());
             CM_HIP(hipStreamSynchronize(stream));
@@ -1825,12 +1835,13 @@ struct Krylov {
     // The whole solve in one resident launch (RsRunner), in apply mode E on
     // systems that were tuned (or come from a one-shot call), which leave the
     // summation order to the engine.  Per pass it took, against the captured
-    // launches, 18 / 45 us at 100^2, 26 / 54 us at 45^3, 40 / 73 us at 64^3 and
-    // 86 / 115 us at 79^3 rows (FP64; FP32 47 / 91 us at 79^3), up to
-    // RS_MAX_ROWS, the most rows whose state the registers hold.  ran = false:
-    // not taken, or the grid could not be resident; x is untouched and the
-    // caller enqueues passes.  Launches being bracketed by profiling events
-    // are the passes', so a profiled solve does not come here.
+    // launches, 18 / 45 us at 100^2, 26 / 54 us at 45^3, 42 / 75 us at 58^3,
+    // 68 / 75 us at 64^3 and 84 / 93 us at 73^3 rows (FP64; FP32 37 / 65 us at
+    // 64^3), up to RS_MAX_ROWS, the most rows whose state the registers of the
+    // CUs hold that it may take.  ran = false: not taken, or the grid could not
+    // be resident; x is untouched and the caller enqueues passes.  Launches
+    // being bracketed by profiling events are the passes', so a profiled solve
+    // does not come here.
     int run_resident(double tol, int NMAX, int info_in, int trace_cap, bool zero_start, SolveState &fin, bool &ran)
     {
         ran = false;

@@ -7,12 +7,13 @@
 // Here every workgroup owns a fixed range of rows, and each thread keeps its
 // R rows' x, r (then s), r0, p, v and M p (then M s), and their values on the
 // matrices' diagonals, in registers for the whole solve.  FP64, per pass: 18
-// us at 100^2 rows (45 launched), 26 us at 45^3 (54), 40 us at 64^3 (73), 86
-// us at 79^3 (115).  What bounds it is the chain of eight exchanges: of the
+// us at 100^2 rows (45 launched), 26 us at 45^3 (54), 42 us at 58^3 (75), 68
+// us at 64^3 (75), 84 us at 73^3 (93); FP32 32 us at 58^3 (62), 46 us at 73^3
+// (75).  What bounds it is the chain of eight exchanges: of the
 // pass at 100^2 rows the gathers of its six products are 6.5 us, the two
 // reductions 5.5, the sums over the diagonals 2, the rest LDS writes, barriers
-// and stores.  Beyond 131072 rows (FP64) the values held spill or are read
-// again.
+// and stores.  With three and four rows per thread (FP64) the values held
+// spill or are read again.
 //
 // Exchange.  Only the vectors that other rows gather go through memory (p,
 // H p, M p and s, H s, M s).  Each entry is its own arrival flag: the buffers
@@ -38,7 +39,7 @@
 // the next read of that buffer.
 //
 // Progress.  Waiting needs every workgroup running at once.  The grid is at
-// most one workgroup per CU, and a workgroup starts working only when all
+// most one workgroup per CU (on some CUs less, rs_room), and a workgroup starts working only when all
 // have arrived: each counts itself in, the first closes the count when the
 // grid is complete or after RS_JOIN_TICKS, and if anyone is missing then all
 // leave; the caller launches the grid again and at last takes the
@@ -55,18 +56,48 @@
 namespace cm {
 
 constexpr int RS_WGS = 256;                // workgroups at most (one per CU)
-constexpr int RS_MAX_ROWS = RS_WGS * 1024 * 2;
+constexpr int RS_MAX_ROWS = RS_WGS / 4 * 3 * 512 * 4;
 constexpr int RS_PER = 8;                  // staged entries per thread and step
 constexpr int RS_STEPS = 16;               // window steps at most (half of them with 1024 threads)
 constexpr int RS_SPINS = 1 << 20;          // loads of one entry before a wait gives up (about a second)
 constexpr int RS_GROUP = 256;              // rows over which the spread of CSR entries is taken
-constexpr double RS_CSR_STEPS = 4.0;       // gather steps of the three products' CSR entries (twice that at the most rows)
+constexpr double RS_CSR_STEPS = 4.0;       // gather steps of the three products' CSR entries
+constexpr int RS_CSR_TWICE = 1 << 19;      // rows on which twice those
 constexpr double RS_CSR_ROW = 256.0;       // entries of the three products' longest CSR rows
 constexpr int RS_TRIES = 16;               // launches of a grid that does not arrive
 constexpr int RS_SKIP = 16;                // launched solves after that
 constexpr long long RS_JOIN_TICKS = 1000000;  // 100 MHz ticks the grid may take to arrive (10 ms)
 constexpr int RS_K = 4;                    // sums per reduction
 constexpr int RS_SETS = 5;                 // reduction slots: setup, alpha and omega of even and odd passes
+
+// CUs that resident grids of this shape may take, so that kernels of other
+// streams go on.  These start on what registers a CU has left, and where a
+// shader engine has room on none of its 8 CUs they wait for the solve to end
+// (dispatch waits for the engine whose turn it is).
+// * FP64 on 512 threads (254 to 256 registers) and FP32 with 4 rows take a CU
+//   whole.  A launched solve of 100^2 rows (2.3 ms alone) beside a loop of such
+//   solves took 3.0 ms next to 216 workgroups, 120 to 340 next to 233 to 256;
+//   one of 110^3 rows (21.5 ms alone) 42, 62 and 115 ms next to 140, 191 and
+//   215, 530 to 1400 next to 233 to 256.  They get three quarters.
+// * FP32 with 2 and 3 rows (218 to 225 registers) leaves room for small
+//   kernels on each CU: 3.3 and 42 to 57 ms next to 245 workgroups, but 22 to
+//   27 and 92 to 115 next to 256.  A CU of each XCD is left.
+// * 256 threads and FP32 with one row (174) leave a third of every CU or
+//   more: 3.2 and 32 ms next to 250 workgroups.
+// grid: workgroups of one grid; whole: they take their CUs whole, and all such
+// grids together get no more; all: grids of any shape together.
+struct RsRoom {
+    int grid, all;
+    bool whole;
+};
+template <class T>
+constexpr RsRoom rs_room(int bsz, int rows, int cus)
+{
+    const bool f64 = sizeof(T) == 8;
+    const int most = cus - cus / 32;
+    if (bsz == 256 || (!f64 && rows == 1)) return {cus, cus, false};
+    return f64 || rows == 4 ? RsRoom{cus - cus / 4, most, true} : RsRoom{most, most, false};
+}
 
 constexpr int rs_steps(int bsz) { return bsz < 1024 ? RS_STEPS : RS_STEPS / 2; }
 
@@ -617,7 +648,7 @@ __device__ __forceinline__ bool rs_join(RsCtl *c, long long ticks, int *sh)
                        wall_clock64() - t0 < ticks) {
                 }
                 const unsigned f = __hip_atomic_fetch_or(&c->join, CLOSED, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-                verdict = f == all ? 1u : 2u;
+                verdict = f == all && ticks > 0 ? 1u : 2u;  // no time at all: never (tests)
                 __hip_atomic_store(&c->verdict, verdict, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
             } else {
                 for (int spin = 0; spin < RS_SPINS; spin++) {

@@ -145,7 +145,7 @@ int cm_system_block_get(cm_system sys, double *X);
  * cm_system_graphs covers the single-RHS solves (which launch kernel by
  * kernel anyway while cm_system_profile brackets launches), and
  * cm_system_block_graphs the block solves.  Solves that run in one launch
- * (tuned systems and blocks of at most 524288 rows) do so in both cases. */
+ * (tuned systems and blocks of at most 393216 rows) do so in both cases. */
 int cm_system_graphs(cm_system sys, int on);
 int cm_system_block_graphs(cm_system sys, int on);
 /* Solves in one launch (resident solves) of this system: taken where they
@@ -213,7 +213,7 @@ int cm_system_block_time_spmm(cm_system sys, char which, int bits, int reps, dou
  * and keeps the fastest.  tiles[6]: the tile choices, 0 for an absent
  * matrix.  Results of later solves are unchanged up to the summation order
  * of the row sums and of the row blocks' partial dot products.  Later
- * single-RHS solves (apply mode E, at most 524288 rows) run in one launch
+ * single-RHS solves (apply mode E, at most 393216 rows) run in one launch
  * where the matrices suit it. */
 int cm_system_autotune(cm_system sys, int reps, int *tiles);
 /* SpMV format of one resident matrix copy: bits 64, 32 or 16 (after

@@ -7,6 +7,7 @@ launch, or by the launched passes from the starting x, each bit for bit what
 it is without the limit.  Solves from several threads wait for their turn and
 give bit for bit what they give alone."""
 import threading
+import time
 
 import numpy as np
 import pytest
@@ -176,3 +177,46 @@ def test_threads_give_what_they_give_alone():
     assert not bad, bad
     for w in work:
         w[0].close()
+
+
+@pytest.mark.parametrize("N,bits", [(58, 64), (64, 64), (63, 32), (64, 32), (73, 32)])
+def test_launched_solves_go_on_beside_resident_ones(N, bits):
+    """A launched solve beside a loop of resident ones finds CUs of its own.
+    Next to a grid on all CUs each of its 500 kernels waited for a solve to
+    end, 60 times its time alone (12 in FP32)."""
+    A, s = _tuned(3, N, "pdfiim")
+    s.set_rhs(cmamd.csr_mv_host(A, cmamd.gen_uniform(3, A.n)))
+    C, small = _tuned(2, 100)
+    small.resident(False)
+    small.set_rhs(cmamd.csr_mv_host(C, cmamd.gen_uniform(5, C.n)))
+
+    if bits != 64:
+        s.enable_mixed(bits)
+        s.autotune(2)
+
+    def once(q):
+        q.set_x(None)
+        t = time.perf_counter()
+        q.solve_mixed(bits, tol=1e-11) if q is s and bits != 64 else q.solve(tol=1e-8)
+        return time.perf_counter() - t
+
+    once(small)
+    alone = np.median([once(small) for _ in range(5)])
+    once(s)
+    c = s.resident(True)
+    stop = threading.Event()
+
+    def loop():
+        while not stop.is_set():
+            once(s)
+
+    th = threading.Thread(target=loop)
+    th.start()
+    time.sleep(0.02)
+    beside = np.median([once(small) for _ in range(5)])
+    stop.set()
+    th.join()
+    assert s.resident(True)[0] > c[0]
+    assert beside <= 5 * alone, (beside, alone)
+    s.close()
+    small.close()
