@@ -199,6 +199,34 @@ static void check_levels(const Csr &A)
     }
 }
 
+// The triangular solve's chunks: every row once, in level order, with its
+// entries; no chunk across two levels; at most three places of the list per row.
+static void check_chunks(const Csr &A)
+{
+    for (bool lower : {true, false}) {
+        const LevelSchedule L = level_schedule(A.n, A.ptr.data(), A.col.data(), lower);
+        const TrsvChunks t = trsv_chunks(L, L.tptr);
+        const std::vector<int> &c = t.row;
+        const int rpw = t.rpc;
+        CHECK(t.lpr >= 1 && t.lpr <= 16 && WAVE % t.lpr == 0 && t.rpc >= 1 && t.rpc <= WAVE / t.lpr, "chunk shape");
+        CHECK(c.size() % (4 * (size_t)rpw) == 0, "whole chunks");
+        CHECK(c.size() <= 12 * (size_t)A.n, "chunk list bounded by the rows");
+        std::vector<int> lev(A.n);
+        for (int l = 0; l < L.nlev; l++)
+            for (int q = L.loff[l]; q < L.loff[l + 1]; q++) lev[L.rows[q]] = l;
+        int q = 0;
+        for (size_t k = 0; k < c.size() / 4; k++) {
+            const int r = c[4 * k], first = c[4 * (k / rpw * rpw)];
+            CHECK(first >= 0, "no empty chunk");
+            if (r < 0) continue;
+            CHECK(q < A.n && r == L.rows[q] && c[4 * k + 1] == L.tptr[q] && c[4 * k + 2] == L.tptr[q + 1], "chunk row");
+            CHECK(first < 0 || lev[first] == lev[r], "chunk of one level");
+            q++;
+        }
+        CHECK(q == A.n, "all rows in chunks");
+    }
+}
+
 static void check_slots(const Csr &A)
 {
     SlotLayout S;
@@ -294,6 +322,7 @@ static void run(const char *name, const Csr &A)
     check_transpose(A);
     check_sym(A);
     check_levels(A);
+    check_chunks(A);
     check_slots(A);
     check_dia(A);
     std::printf("%-28s n=%7d nnz=%9zu %s\n", name, A.n, A.col.size(), g_fail == before ? "ok" : "FAILED");
@@ -327,6 +356,14 @@ int main()
         }
         run("upper triangular", from_rows(R.n, up));
         run("lower triangular", from_rows(R.n, lo));
+    }
+    for (int w : {1, 2, 3, 63, 65}) {  // w rows per level, each reading one of the level before
+        std::vector<std::set<int>> rows(4000);
+        for (int i = 0; i < 4000; i++) {
+            rows[i].insert(i);
+            if (i >= w) rows[i].insert(i - w);
+        }
+        run("levels of few rows", from_rows(4000, rows));
     }
     if (g_fail) {
         std::fprintf(stderr, "%d check(s) failed\n", g_fail);

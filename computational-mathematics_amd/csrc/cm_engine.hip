@@ -458,8 +458,8 @@ struct DevCsr {
     bool lower = false;  // the level schedule's triangle (lower: rows read smaller columns)
     int *lrows = nullptr;
     int nchunk = 0;
-    int4 *crow = nullptr;  // the triangular solve's chunks: nchunk x (WAVE / lpr) of {row, first entry, end, 0}
-    int lpr = 1;          // lanes per row of the triangular solve
+    int4 *crow = nullptr;  // the triangular solve's chunks: nchunk x rpc of {row or -1, first entry, end, 0}
+    int lpr = 1, rpc = 1;  // its lanes per row and rows per chunk
     // the triangle's entries in level order (tptr indexed by level position;
     // tsrc: CSR positions; tval: this copy's values gathered through tsrc)
     int *tptr = nullptr, *tcol = nullptr, *tsrc = nullptr;
@@ -479,7 +479,7 @@ struct DevCsr {
             if (slots) b += slots->bytes();
             if (dia) b += dia->bytes();
             b += (size_t)(n + 1 + 2 * (nblk + 1)) * sizeof(int) + (size_t)nnz * sizeof(int) + (lrows ? (size_t)n * sizeof(int) : 0);
-            if (crow) b += (size_t)nchunk * (WAVE / lpr) * sizeof(int4);
+            if (crow) b += (size_t)nchunk * rpc * sizeof(int4);
             if (d16) b += (size_t)(nnz + 2 * CSR_PAD) * sizeof(uint16_t) + (size_t)nblk * sizeof(int);
         }
         return b;
@@ -592,6 +592,7 @@ static int cast_csr(DevCsr<V> &dst, const DevCsr<double> &src, hipStream_t s)
     dst.crow = src.crow;
     dst.nchunk = src.nchunk;
     dst.lpr = src.lpr;
+    dst.rpc = src.rpc;
     dst.tptr = src.tptr;
     dst.tcol = src.tcol;
     dst.tsrc = src.tsrc;
@@ -1033,16 +1034,11 @@ static int build_levels(DevCsr<double> &m, const int *ptr, const int *col, bool 
     CM_TRY(dev_alloc(&m.tval, (size_t)m.ntri));
     k_tri_fill<<<g, BS, 0, s>>>(n, m.lrows, m.ptr, m.col, lower, m.tptr, m.tcol, m.tsrc);
     if (m.ntri) k_gather_vals<double><<<long_grid(m.ntri), BS, 0, s>>>(m.ntri, m.tsrc, m.val, m.tval);
-    m.lpr = trsv_lanes((double)m.ntri / m.n);
-    // chunks of one wave's rows, none across two levels (padded with row -1)
-    const int rpw = WAVE / m.lpr;
-    std::vector<int4> crow;
-    for (int l = 0; l < L.nlev; l++) {
-        for (int q = L.loff[l]; q < L.loff[l + 1]; q++) crow.push_back(make_int4(L.rows[q], tp[q], tp[q + 1], 0));
-        while (crow.size() % rpw) crow.push_back(make_int4(-1, 0, 0, 0));
-    }
-    m.nchunk = (int)(crow.size() / rpw);
-    CM_TRY(dev_upload(&m.crow, crow.data(), crow.size(), s));
+    const TrsvChunks chunks = trsv_chunks(L, tp);
+    m.lpr = chunks.lpr;
+    m.rpc = chunks.rpc;
+    m.nchunk = (int)(chunks.row.size() / 4 / m.rpc);
+    CM_TRY(dev_upload(&m.crow, reinterpret_cast<const int4 *>(chunks.row.data()), chunks.row.size() / 4, s));
     CM_HIP(hipGetLastError());
     CM_HIP(hipStreamSynchronize(s));  // before the temporaries are freed
     return CM_OK;
@@ -1708,7 +1704,7 @@ struct Krylov {
                 // waves for two and a half levels' chunks
                 const long long waves = std::min<long long>(512, 5LL * m.nchunk / (2LL * std::max(1, m.nlev)) + 4);
                 const int g = (int)(TRSV_XCDS * ((waves + TRSV_BS / WAVE - 1) / (TRSV_BS / WAVE)));
-                k_trsv_flow<T, VF, LPR><<<g, TRSV_BS, 0, stream>>>(m.nchunk, m.crow, m.tcol, m.tval, m.rowscale,
+                k_trsv_flow<T, VF, LPR><<<g, TRSV_BS, 0, stream>>>(m.nchunk, m.rpc, m.crow, m.tcol, m.tval, m.rowscale,
                                                                   bin, dscale, xout, trsv_ctl + q,
                                                                   use_state ? st : nullptr, use_state ? st : nullptr);
             };

@@ -31,7 +31,6 @@
 namespace cm {
 
 constexpr int TRSV_BS = 256;
-constexpr int TRSV_P = 4;  // entries per lane loaded ahead of the chunk's turn
 
 struct TrsvCtl {  // cleared (xcd: -1) by k_trsv_prep
     int ticket;
@@ -61,14 +60,6 @@ __global__ __launch_bounds__(BS) void k_trsv_prep(int n, T *__restrict__ x0, T *
     }
 }
 
-// Lanes per row: enough for the mean row to be loaded ahead, a power of two.
-inline int trsv_lanes(double mean)
-{
-    int l = 1;
-    while (l < 16 && TRSV_P * l < mean) l *= 2;
-    return l;
-}
-
 // One chunk's row as a lane sees it: LPR lanes per row, lane l holds the
 // row's entries l, l + LPR, ...
 struct TrsvRow {
@@ -82,8 +73,8 @@ struct TrsvRow {
 // chunk order: x[i] = (b[i] - sum_{j != i} T[i,j] x[j]) / T[i,i], T[i,i] = 1
 // when the row stores no diagonal.  Only the declared triangle's entries are
 // stored there, as the TRIANGULAR descriptor makes mkl_sparse_d_trsv read
-// (ACIFIM/src/bicgstab.cpp:170-176).  Chunk c's rows are crow[c * WAVE / LPR
-// ..], all of one level.  dscale (or null): b is taken as b .* dscale,
+// (ACIFIM/src/bicgstab.cpp:170-176).  Chunk c's rows are crow[c * rpc ..],
+// rpc <= WAVE / LPR, all of one level.  dscale (or null): b is taken as b .* dscale,
 // rounded to T (the D^-1 between the two solves of mode I).  Three chunks are
 // under way in a wave: the rows of the third are being read, the entries and
 // right-hand sides of the second, and the first waits for x, so no load but
@@ -91,7 +82,7 @@ struct TrsvRow {
 // us per chunk, mostly on the three dependent loads).  rep: told when a wait
 // is given up.
 template <class T, class V, int LPR>
-__global__ __launch_bounds__(TRSV_BS) void k_trsv_flow(int chunks, const int4 *__restrict__ crow,
+__global__ __launch_bounds__(TRSV_BS) void k_trsv_flow(int chunks, int rpc, const int4 *__restrict__ crow,
                                                        const int *__restrict__ tcol, const V *__restrict__ tval,
                                                        const float *__restrict__ rowscale, const T *__restrict__ b,
                                                        const T *__restrict__ dscale, T *x, TrsvCtl *c,
@@ -119,7 +110,7 @@ __global__ __launch_bounds__(TRSV_BS) void k_trsv_flow(int chunks, const int4 *_
         return t;
     };
     auto rows = [&](int chunk) {  // chunk past the last: no rows
-        return chunk < chunks ? crow[(size_t)chunk * (WAVE / LPR) + g] : make_int4(-1, 0, 0, 0);
+        return chunk < chunks && g < rpc ? crow[(size_t)chunk * rpc + g] : make_int4(-1, 0, 0, 0);
     };
     auto fetch = [&](TrsvRow &rw) {
         const int i = rw.at.x;
