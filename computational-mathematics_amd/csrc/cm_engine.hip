@@ -460,6 +460,7 @@ struct DevCsr {
     int nchunk = 0;
     int4 *crow = nullptr;  // the triangular solve's chunks: nchunk x rpc of {row or -1, first entry, end, 0}
     int lpr = 1, rpc = 1;  // its lanes per row and rows per chunk
+    std::vector<int> loff;  // the levels' first rows in level order, where each level is a launch of its own
     // the triangle's entries in level order (tptr indexed by level position;
     // tsrc: CSR positions; tval: this copy's values gathered through tsrc)
     int *tptr = nullptr, *tcol = nullptr, *tsrc = nullptr;
@@ -593,6 +594,7 @@ static int cast_csr(DevCsr<V> &dst, const DevCsr<double> &src, hipStream_t s)
     dst.nchunk = src.nchunk;
     dst.lpr = src.lpr;
     dst.rpc = src.rpc;
+    dst.loff = src.loff;
     dst.tptr = src.tptr;
     dst.tcol = src.tcol;
     dst.tsrc = src.tsrc;
@@ -1034,11 +1036,19 @@ static int build_levels(DevCsr<double> &m, const int *ptr, const int *col, bool 
     CM_TRY(dev_alloc(&m.tval, (size_t)m.ntri));
     k_tri_fill<<<g, BS, 0, s>>>(n, m.lrows, m.ptr, m.col, lower, m.tptr, m.tcol, m.tsrc);
     if (m.ntri) k_gather_vals<double><<<long_grid(m.ntri), BS, 0, s>>>(m.ntri, m.tsrc, m.val, m.tval);
-    const TrsvChunks chunks = trsv_chunks(L, tp);
-    m.lpr = chunks.lpr;
-    m.rpc = chunks.rpc;
-    m.nchunk = (int)(chunks.row.size() / 4 / m.rpc);
-    CM_TRY(dev_upload(&m.crow, reinterpret_cast<const int4 *>(chunks.row.data()), chunks.row.size() / 4, s));
+    m.loff.clear();
+    TrsvChunks chunks;
+    if (n > (long long)TRSV_LEVEL_ROWS * L.nlev) {  // launches of whole levels, a lane per entry of the mean row
+        m.loff = L.loff;
+        m.lpr = 1;
+        while (m.lpr < 16 && m.lpr < (double)m.ntri / n) m.lpr *= 2;
+    } else {
+        chunks = trsv_chunks(L, tp);
+        m.lpr = chunks.lpr;
+        m.rpc = chunks.rpc;
+        m.nchunk = (int)(chunks.row.size() / 4 / m.rpc);
+        CM_TRY(dev_upload(&m.crow, reinterpret_cast<const int4 *>(chunks.row.data()), chunks.row.size() / 4, s));
+    }
     CM_HIP(hipGetLastError());
     CM_HIP(hipStreamSynchronize(s));  // before the temporaries are freed
     return CM_OK;
@@ -1520,7 +1530,10 @@ struct Krylov {
         const int maxblk = std::max(nblk_a, MAX_RED_BLOCKS);
         CM_HIP(hipMalloc((void **)&partials, (size_t)maxblk * 4 * sizeof(double)));
         partials_cap = (size_t)maxblk * 4;
-        if (variant == 2 && (mode == 'I' || mode == 'J')) CM_TRY(dev_alloc(&trsv_ctl, 2));
+        if (variant == 2 && (mode == 'I' || mode == 'J')) {
+            CM_TRY(dev_alloc(&trsv_ctl, 2));
+            CM_HIP(hipMemsetAsync(trsv_ctl, 0, 2 * sizeof(TrsvCtl), stream));
+        }
         for (auto &e : ev) CM_HIP(hipEventCreateWithFlags(&e, hipEventDisableTiming));
         return CM_OK;
     }
@@ -1691,7 +1704,7 @@ struct Krylov {
     }
 
     // x = T^{-1} (b .* dscale) for a triangular factor in level order (dscale
-    // null: T^{-1} b); the q-th of the pair that trsv_prep readied
+    // null: T^{-1} b); the q-th of the pair that k_trsv_prep readied
     void trsv(const DevCsr<VF> &m, const T *bin, const T *dscale, T *xout, int q, bool use_state)
     {
         // the triangle's entries (value + column), row list and row pointers once, and per row
@@ -1701,6 +1714,16 @@ struct Krylov {
         timed(KC_LU, by, [&] {
             auto go = [&](auto lz) {
                 constexpr int LPR = decltype(lz)::value;
+                if (!m.loff.empty()) {
+                    for (size_t l = 0; l + 1 < m.loff.size(); l++) {
+                        const int q0 = m.loff[l], cnt = m.loff[l + 1] - q0;
+                        const int g = (int)(((long long)cnt * LPR + BS - 1) / BS);
+                        k_trsv_level<T, VF, LPR><<<g, BS, 0, stream>>>(cnt, m.lrows + q0, m.tptr + q0, m.tcol, m.tval,
+                                                                       m.rowscale, bin, dscale, xout,
+                                                                       use_state ? st : nullptr);
+                    }
+                    return;
+                }
                 // waves for two and a half levels' chunks
                 const long long waves = std::min<long long>(512, 5LL * m.nchunk / (2LL * std::max(1, m.nlev)) + 4);
                 const int g = (int)(TRSV_XCDS * ((waves + TRSV_BS / WAVE - 1) / (TRSV_BS / WAVE)));
@@ -1730,7 +1753,7 @@ struct Krylov {
         }
         if (mode == 'I' || mode == 'J') {
             // I: t1 = L^{-1} b; x = U^{-1} (t1 .* IDv).   J: x = U^{-1} L^{-1} b.
-            timed(KC_VEC, 2.0 * sizeof(T) * n, [&] {
+            if (L.loff.empty() || U.loff.empty()) timed(KC_VEC, 2.0 * sizeof(T) * n, [&] {
                 k_trsv_prep<T><<<vec_grid(n), BS, 0, stream>>>(n, t1, out, trsv_ctl, use_state ? st : nullptr);
             });
             trsv(L, in, nullptr, t1, 0, use_state);

@@ -1,6 +1,7 @@
 // Sparse triangular solves (ACIFIM apply modes 'I' and 'J',
 // ACIFIM/src/bicgstab.cpp:405-406,421-427: mkl_sparse_d_trsv on the unit
-// triangular L and U with their stored diagonal), one launch per triangle.
+// triangular L and U with their stored diagonal): one launch per triangle, or
+// one per level where levels are wide (k_trsv_level).
 //
 // The host orders the rows by dependency level once per factor (a row's level
 // is one more than the deepest row it reads), stores the triangle's entries
@@ -25,12 +26,20 @@
 // stores, which go on to memory, and 6.5 us for a kernel boundary per level.
 // A level so takes 1.1 us up to 64^3 rows and 1.9 us at 128^3.
 // The first workgroup to arrive fixes the XCD; the others leave.
+//
+// One XCD reads an eighth of what the device does, so a level of w rows takes
+// about 1 + 0.4 w/1000 us here and 3.3 + 0.04 w/1000 us as a launch on all
+// CUs (2^20 rows of four entries, L and U, us per apply, here / launches: 256
+// levels 1430 / 1725, 128 levels 1070 / 890, 64 levels 1110 / 470, 16 levels
+// 530 / 180, one level 465 / 57).  Summed over the levels the two are equal
+// where the mean level has some 6000 rows: TRSV_LEVEL_ROWS.
 #pragma once
 #include "cm_resident.hpp"
 
 namespace cm {
 
 constexpr int TRSV_BS = 256;
+constexpr int TRSV_LEVEL_ROWS = 6000;  // mean rows per level beyond which each level is a launch
 
 struct TrsvCtl {  // cleared (xcd: -1) by k_trsv_prep
     int ticket;
@@ -58,6 +67,42 @@ __global__ __launch_bounds__(BS) void k_trsv_prep(int n, T *__restrict__ x0, T *
         c[t0].xcd = -1;
         c[t0].fail = 0;
     }
+}
+
+// One level of a triangular solve, the rows rows[0 .. cnt) with the entries
+// tptr[q] .. tptr[q + 1] of row q: x[i] = (b[i] - sum_{j != i} T[i,j] x[j]) /
+// T[i,i], as k_trsv_flow below, the rows it reads being there from the
+// launches before.  LPR lanes per row, lane l takes its entries l, l + LPR, ...
+// Bound by memory: a level of 2^20 rows of one entry takes 14 us, 44 MB.
+template <class T, class V, int LPR>
+__global__ __launch_bounds__(BS) void k_trsv_level(int cnt, const int *__restrict__ rows, const int *__restrict__ tptr,
+                                                   const int *__restrict__ tcol, const V *__restrict__ tval,
+                                                   const float *__restrict__ rowscale, const T *__restrict__ b,
+                                                   const T *__restrict__ dscale, T *x, const SolveState *st)
+{
+    if (st && st->done) return;
+    const int q = (int)((blockIdx.x * (unsigned)BS + threadIdx.x) / LPR), l = (int)(threadIdx.x % LPR);
+    if (q >= cnt) return;  // the row's LPR lanes leave together
+    const int i = rows[q], e = tptr[q + 1];
+    const double sc = rowscale ? (double)rowscale[i] : 1.0;
+    double s = 0.0, d = 0.0, hasd = 0.0;
+    for (int k = tptr[q] + l; k < e; k += LPR) {
+        const int j = tcol[k];
+        const double a = load_val<V, double>(tval, k) * sc;
+        if (j == i) {
+            d = a;
+            hasd = 1.0;
+        } else {
+            s += a * (double)x[j];
+        }
+    }
+#pragma unroll
+    for (int o = LPR / 2; o > 0; o >>= 1) {
+        s += __shfl_xor(s, o, LPR);
+        d += __shfl_xor(d, o, LPR);
+        hasd += __shfl_xor(hasd, o, LPR);
+    }
+    if (l == 0) x[i] = (T)(((dscale ? (double)(b[i] * dscale[i]) : (double)b[i]) - s) / (hasd > 0.0 ? d : 1.0));
 }
 
 // One chunk's row as a lane sees it: LPR lanes per row, lane l holds the
