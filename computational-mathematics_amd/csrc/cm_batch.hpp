@@ -13,9 +13,10 @@
 // the counter passes the item count, and every solve ends by NMAX, so the
 // grid always drains.
 //
-// Systems of at most BT_ROWS rows run in k_batch_small, which keeps the
-// vectors in LDS and registers and streams the matrices through LDS; the rest
-// of this comment is k_batch_solve, for larger ones.
+// Systems of at most BT_ROWS rows and bt_mean entries per row run in
+// k_batch_small, which keeps the vectors in LDS and registers and streams the
+// matrices through LDS; the rest of this comment is k_batch_solve, for the
+// others.
 // Per workgroup: SpMV rows go to groups of LPR lanes (xor-shuffle sums inside
 // the group); vector updates stride over the rows; dot products and norms
 // are summed in a fixed order (per-thread, wave shuffles, then the waves in
@@ -229,7 +230,8 @@ __device__ void wg_bicgstab(const BatchSys &S, BatchItem &it, double *w, double 
     }
 }
 
-// ---- systems of at most BT_ROWS rows: vectors in LDS and registers
+// ---- systems of at most BT_ROWS rows (and bt_mean entries per row): vectors in
+// LDS and registers
 //
 // A pass is bound by reading the matrices (12 bytes per entry): one CU holds
 // some 60 reads in flight, which from the L2 and the MALL gives it about 20
@@ -245,7 +247,9 @@ __device__ void wg_bicgstab(const BatchSys &S, BatchItem &it, double *w, double 
 constexpr int BT_BS = 512;    // threads: 8 waves, which leaves a thread 256 registers (1024 threads spilled)
 constexpr int BT_PER = 16;
 constexpr int BT_TILE = BT_PER * BT_BS;
-constexpr int BT_ROWS = 4096;  // two vectors of them and a tile fill the LDS
+constexpr int BT_ROWS = 4096;  // two vectors of them and a tile take 132 of the LDS's 160 KB
+// entries per row of a matrix, on the mean, up to which this kernel is the faster one
+constexpr int bt_mean(int n) { return n <= 2 * BT_BS ? 80 : 170; }
 
 using BatchSysTable = RsConst<BatchSys>;  // the tables are written before the launch
 
@@ -541,7 +545,8 @@ __device__ __forceinline__ void bt_bicgstab(BatchSysTable S, RsConst<BatchItem> 
 // LDS of k_batch_small, in doubles: tile, two vectors, sums.
 constexpr int BT_LDS = BT_TILE + 2 * BT_ROWS + 3 * 32;
 
-// The queue of k_batch_solve for items whose systems have at most BT_ROWS rows.
+// The queue of k_batch_solve for items whose systems have at most BT_ROWS rows
+// (rows of any length).
 __global__ __launch_bounds__(BT_BS) void k_batch_small(int nitems, const BatchSys *__restrict__ sys, BatchItem *items,
                                                        double *arena, size_t slot_stride, int *head, int restart_true)
 {

@@ -3384,8 +3384,22 @@ static BatchSys batch_sys(const K64 &k)
                     {H.col, k.G.col, k.A.col}, {H.val, k.G.val, k.A.val}, k.idv};
 }
 
-// The two kernels over items sorted by size, largest first: the first nl are
-// beyond k_batch_small's LDS.  head: two ints.
+// Items for k_batch_small: their vectors fit its LDS, and no matrix has so many
+// entries per row that one thread per row is slower than k_batch_solve's eight
+// lanes.  64 items, us per pass here / there: 500 rows of 30, 70, 83 and 276
+// entries 22 / 33, 45 / 45, 54 / 50 and 258 / 101; 1000 rows of 87 and 114
+// 94 / 92 and 128 / 105; 2000 rows of 60, 155, 236 and 443 entries 115 / 146,
+// 372 / 404, 698 / 566 and 2110 / 971; 4096 rows of 61, 158, 187 and 225
+// 234 / 432, 787 / 844, 992 / 987 and 1329 / 1153.  A few long rows among short
+// ones are no loss (three of 4000 entries in 4000 rows 283 / 313).
+static bool batch_small(const K64 &k)
+{
+    const long long most = std::max({k.A.nnz, k.G.nnz, (k.sym ? k.GT : k.H).nnz});
+    return k.n <= BT_ROWS && most <= (long long)bt_mean(k.n) * k.n;
+}
+
+// The two kernels over sorted items, the first nl for k_batch_solve.  head:
+// two ints.
 static int launch_batch(int nitems, int nl, int grid, const BatchSys *dsys, BatchItem *ditems, double *arena,
                         size_t stride, int *head, int restart_true, hipStream_t s)
 {
@@ -3454,11 +3468,14 @@ struct BatchRunner {
             hs[q] = batch_sys(k);
             maxn = std::max(maxn, k.n);
         }
-        // largest systems first (longest solves start early)
+        // k_batch_solve's first, then largest systems first (longest solves start early)
         std::vector<int> order(nitems);
         for (int i = 0; i < nitems; i++) order[i] = i;
-        std::stable_sort(order.begin(), order.end(),
-                         [&](int a, int b) { return systems[sys_of[a]]->n > systems[sys_of[b]]->n; });
+        std::stable_sort(order.begin(), order.end(), [&](int a, int b) {
+            const K64 &ka = *systems[sys_of[a]]->k64, &kb = *systems[sys_of[b]]->k64;
+            const bool sa = batch_small(ka), sb = batch_small(kb);
+            return sa != sb ? sb : ka.n > kb.n;
+        });
         // vec: all right-hand sides, then all solutions, each in item order
         std::vector<size_t> off(nitems);
         size_t half = 0;
@@ -3510,8 +3527,8 @@ struct BatchRunner {
         if (staged) CM_HIP(hipMemcpyAsync(vec, hvec, tot * sizeof(double), hipMemcpyHostToDevice, s));
         CM_HIP(hipMemcpyAsync(dsys, hs.data(), ns * sizeof(BatchSys), hipMemcpyHostToDevice, s));
         CM_HIP(hipMemcpyAsync(ditems, hitems, (size_t)nitems * sizeof(BatchItem), hipMemcpyHostToDevice, s));
-        int nl = 0;  // items too large for k_batch_small come first
-        while (nl < nitems && systems[sys_of[order[nl]]]->n > BT_ROWS) nl++;
+        int nl = 0;
+        while (nl < nitems && !batch_small(*systems[sys_of[order[nl]]]->k64)) nl++;
         CM_TRY(launch_batch(nitems, nl, grid, dsys, ditems, arena, stride, head, restart_true, s));
         CM_HIP(hipMemcpyAsync(hitems, ditems, (size_t)nitems * sizeof(BatchItem), hipMemcpyDeviceToHost, s));
         if (staged) CM_HIP(hipMemcpyAsync(hvec + half, vec + half, half * sizeof(double), hipMemcpyDeviceToHost, s));
@@ -4068,11 +4085,13 @@ int cm_batch_solve_noalloc(int nitems, const cm_system *systems, const double *c
                                     " rows needs more than the " + std::to_string(NA_ARENA_BYTES >> 20) +
                                     " MiB work arena");
     const int grid = (int)std::min<size_t>({(size_t)nitems, (size_t)cus, slots});
-    // largest systems first; ties in item order
+    // k_batch_solve's first, then largest systems first; ties in item order
     for (int i = 0; i < nitems; i++) g_na_order[i] = i;
     std::sort(g_na_order, g_na_order + nitems, [](int a, int b) {
-        const int na = g_na_sysptr[g_na_sys_of[a]]->n, nb = g_na_sysptr[g_na_sys_of[b]]->n;
-        return na != nb ? na > nb : a < b;
+        const K64 &ka = *g_na_sysptr[g_na_sys_of[a]]->k64, &kb = *g_na_sysptr[g_na_sys_of[b]]->k64;
+        const bool sa = batch_small(ka), sb = batch_small(kb);
+        if (sa != sb) return sb;
+        return ka.n != kb.n ? ka.n > kb.n : a < b;
     });
     for (int q = 0; q < nitems; q++) {
         const int i = g_na_order[q];
@@ -4085,8 +4104,8 @@ int cm_batch_solve_noalloc(int nitems, const cm_system *systems, const double *c
     double *arena = reinterpret_cast<double *>(base + NA_ARENA);
     CM_HIP(hipMemcpyAsync(dsys, g_na_sys, ns * sizeof(BatchSys), hipMemcpyHostToDevice, s));
     CM_HIP(hipMemcpyAsync(ditems, g_na_items, (size_t)nitems * sizeof(BatchItem), hipMemcpyHostToDevice, s));
-    int nl = 0;  // items too large for k_batch_small come first
-    while (nl < nitems && g_na_sysptr[g_na_items[nl].sys]->n > BT_ROWS) nl++;
+    int nl = 0;
+    while (nl < nitems && !batch_small(*g_na_sysptr[g_na_items[nl].sys]->k64)) nl++;
     CM_TRY(launch_batch(nitems, nl, grid, dsys, ditems, arena, stride, head, restart_true, s));
     CM_HIP(hipMemcpyAsync(g_na_items, ditems, (size_t)nitems * sizeof(BatchItem), hipMemcpyDeviceToHost, s));
     CM_HIP(hipStreamSynchronize(s));
