@@ -3398,17 +3398,34 @@ static bool batch_small(const K64 &k)
     return k.n <= BT_ROWS && most <= (long long)bt_mean(k.n) * k.n;
 }
 
-// The two kernels over sorted items, the first nl for k_batch_solve.  head:
-// two ints.
+// The work vectors of a batch: doubles per workgroup of k_batch_solve (n_max
+// rows) and of k_batch_small.
+static size_t batch_stride(int maxn) { return ((size_t)9 * maxn + 63) / 64 * 64; }
+constexpr size_t BT_STRIDE = BT_ROWS + 64;  // not a power of two apart
+
+// The two kernels over sorted items, the first nl for k_batch_solve, on at most
+// `grid` workgroups each (one fits a CU).  head: two ints.  The large items
+// are launched first.  side (or null): the small ones run beside them on that
+// stream, on the CUs the large ones leave (e: two events); else behind them.
+// 200 items of 20^3 rows (12.1 ms) and 200 of 400 to 3600 (3.3 ms): 15.5 ms one
+// behind the other, 13.7 so; 24 of 30^3 and 232 small ones 48.9 and 46.9.  arena: of k_batch_solve's workgroups; small: of k_batch_small's.
 static int launch_batch(int nitems, int nl, int grid, const BatchSys *dsys, BatchItem *ditems, double *arena,
-                        size_t stride, int *head, int restart_true, hipStream_t s)
+                        size_t stride, double *small, size_t small_stride, int *head, int restart_true, hipStream_t s,
+                        hipStream_t side, const hipEvent_t *e)
 {
+    const int ns = nitems - nl;
     k_zero_int<<<1, 2, 0, s>>>(head);
+    if (side) CM_HIP(hipEventRecord(e[0], s));
     if (nl > 0)
         k_batch_solve<<<std::min(grid, nl), PBS, 0, s>>>(nl, dsys, ditems, arena, stride, head, restart_true);
-    const int ns = nitems - nl;
+    if (side) CM_HIP(hipStreamWaitEvent(side, e[0], 0));
     if (ns > 0)
-        k_batch_small<<<std::min(grid, ns), BT_BS, 0, s>>>(ns, dsys, ditems + nl, arena, stride, head + 1, restart_true);
+        k_batch_small<<<std::min(grid, ns), BT_BS, 0, side ? side : s>>>(ns, dsys, ditems + nl, small, small_stride,
+                                                                        head + 1, restart_true);
+    if (side) {
+        CM_HIP(hipEventRecord(e[1], side));
+        CM_HIP(hipStreamWaitEvent(s, e[1], 0));
+    }
     CM_HIP(hipGetLastError());
     return CM_OK;
 }
@@ -3426,8 +3443,13 @@ struct BatchRunner {
     double *hvec = nullptr;  // pinned, at most STAGE_MAX bytes
     size_t hvec_cap = 0;
     static constexpr size_t STAGE_MAX = (size_t)64 << 20;
+    hipStream_t side = nullptr;  // the small items' beside large ones, made on first use
+    hipEvent_t ev[2] = {nullptr, nullptr};
     ~BatchRunner()
     {
+        for (auto &e : ev)
+            if (e) (void)hipEventDestroy(e);
+        if (side) (void)hipStreamDestroy(side);
         if (hvec) (void)hipHostFree(hvec);
         (void)hipFree(dsys);
         (void)hipFree(ditems);
@@ -3439,6 +3461,12 @@ struct BatchRunner {
     size_t bytes() const
     {
         return sys_cap * sizeof(BatchSys) + item_cap * sizeof(BatchItem) + (arena_cap + vec_cap) * sizeof(double);
+    }
+
+    // doubles of work vectors for nl and ns items of the two kernels
+    static size_t arena_need(int nl, int ns, int maxn, int cus)
+    {
+        return batch_stride(maxn) * std::min(nl, cus) + BT_STRIDE * std::min(ns, cus);
     }
 
     template <class P>
@@ -3487,8 +3515,15 @@ struct BatchRunner {
         int dev = 0, cus = 256;
         CM_HIP(hipGetDevice(&dev));
         CM_HIP(hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev));
-        const int grid = std::min(nitems, cus);  // one PBS-thread workgroup fits a CU
-        const size_t stride = ((size_t)9 * maxn + 63) / 64 * 64;
+        const int grid = std::min(nitems, cus);
+        const size_t stride = batch_stride(maxn);
+        int nl = 0;
+        while (nl < nitems && !batch_small(*systems[sys_of[order[nl]]]->k64)) nl++;
+        const bool both = nl > 0 && nl < nitems;
+        if (both && !side) {
+            CM_HIP(hipStreamCreateWithFlags(&side, hipStreamNonBlocking));
+            for (auto &e : ev) CM_HIP(hipEventCreateWithFlags(&e, hipEventDisableTiming));
+        }
         CM_TRY(grow(&dsys, sys_cap, (size_t)ns));
         CM_TRY(grow(&ditems, item_cap, (size_t)nitems));
         if (nitems > (int)hitems_cap) {
@@ -3497,7 +3532,7 @@ struct BatchRunner {
             CM_HIP(hipHostMalloc((void **)&hitems, (size_t)nitems * sizeof(BatchItem), hipHostMallocDefault));
             hitems_cap = nitems;
         }
-        CM_TRY(grow(&arena, arena_cap, stride * grid));
+        CM_TRY(grow(&arena, arena_cap, arena_need(nl, nitems - nl, maxn, cus)));
         CM_TRY(grow(&vec, vec_cap, tot));
         if (!head) CM_HIP(hipMalloc((void **)&head, 2 * sizeof(int)));
         // the vectors cross in one copy each way through pinned memory where
@@ -3527,9 +3562,8 @@ struct BatchRunner {
         if (staged) CM_HIP(hipMemcpyAsync(vec, hvec, tot * sizeof(double), hipMemcpyHostToDevice, s));
         CM_HIP(hipMemcpyAsync(dsys, hs.data(), ns * sizeof(BatchSys), hipMemcpyHostToDevice, s));
         CM_HIP(hipMemcpyAsync(ditems, hitems, (size_t)nitems * sizeof(BatchItem), hipMemcpyHostToDevice, s));
-        int nl = 0;
-        while (nl < nitems && !batch_small(*systems[sys_of[order[nl]]]->k64)) nl++;
-        CM_TRY(launch_batch(nitems, nl, grid, dsys, ditems, arena, stride, head, restart_true, s));
+        CM_TRY(launch_batch(nitems, nl, grid, dsys, ditems, arena, stride, arena + stride * std::min(nl, grid), BT_STRIDE,
+                            head, restart_true, s, both ? side : nullptr, ev));
         CM_HIP(hipMemcpyAsync(hitems, ditems, (size_t)nitems * sizeof(BatchItem), hipMemcpyDeviceToHost, s));
         if (staged) CM_HIP(hipMemcpyAsync(hvec + half, vec + half, half * sizeof(double), hipMemcpyDeviceToHost, s));
         else
@@ -4078,7 +4112,7 @@ int cm_batch_solve_noalloc(int nitems, const cm_system *systems, const double *c
         }
         g_na_sys_of[i] = q;
     }
-    const size_t stride = ((size_t)9 * maxn + 63) / 64 * 64;  // doubles per workgroup
+    const size_t stride = batch_stride(maxn);  // doubles per workgroup
     const size_t slots = NA_ARENA_BYTES / (stride * sizeof(double));
     if (slots < 1)
         return fail(CM_ERR_ARG, "cm_batch_solve_noalloc: a system of " + std::to_string(maxn) +
@@ -4106,7 +4140,8 @@ int cm_batch_solve_noalloc(int nitems, const cm_system *systems, const double *c
     CM_HIP(hipMemcpyAsync(ditems, g_na_items, (size_t)nitems * sizeof(BatchItem), hipMemcpyHostToDevice, s));
     int nl = 0;
     while (nl < nitems && !batch_small(*g_na_sysptr[g_na_items[nl].sys]->k64)) nl++;
-    CM_TRY(launch_batch(nitems, nl, grid, dsys, ditems, arena, stride, head, restart_true, s));
+    CM_TRY(launch_batch(nitems, nl, grid, dsys, ditems, arena, stride, arena, stride, head, restart_true, s, nullptr,
+                        nullptr));
     CM_HIP(hipMemcpyAsync(g_na_items, ditems, (size_t)nitems * sizeof(BatchItem), hipMemcpyDeviceToHost, s));
     CM_HIP(hipStreamSynchronize(s));
     for (int q = 0; q < nitems; q++) {

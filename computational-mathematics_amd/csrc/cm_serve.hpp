@@ -143,15 +143,16 @@ struct Server {
     // Device bytes worker w's batch runner would add for these requests.
     size_t persistent_need(int w, const std::vector<Request *> &reqs_) const
     {
-        size_t cols = 0, vec = 0;
+        size_t cols = 0, large = 0, vec = 0;
         int maxn = 0;
         for (const Request *r : reqs_) {
             const int n = systems[r->sys].sys->n;
             cols += r->k;
+            if (!batch_small(*systems[r->sys].sys->k64)) large += r->k;
             vec += 2 * (size_t)n * r->k;
             maxn = std::max(maxn, n);
         }
-        const size_t arena = std::min(cols, (size_t)cus) * ((9 * (size_t)maxn + 63) / 64 * 64);
+        const size_t arena = BatchRunner::arena_need((int)large, (int)(cols - large), maxn, cus);
         const size_t want = (arena + vec) * sizeof(double) + cols * sizeof(BatchItem) + systems.size() * sizeof(BatchSys);
         return want > runner_bytes[w] ? want - runner_bytes[w] : 0;
     }

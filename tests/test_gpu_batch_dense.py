@@ -2,6 +2,8 @@
 the line (80 on the mean, 170 beyond 1024 rows) where they change kernels, in one call with sparse
 and with large systems.  Bars are the FP64 path's: info equal, pass counts
 within 2%, x within 1e-7 of the oracle's (a dozen passes)."""
+import threading
+
 import numpy as np
 import pytest
 import scipy.sparse as sp
@@ -48,3 +50,29 @@ def test_batch_by_entries_per_row():
     for r, (xo, rvo, ito, info_o, _) in zip(cmamd.batch_solve(batch), want):
         assert r.info == info_o and abs(r.iter - ito) <= max(1, int(np.ceil(0.02 * ito)))
         assert np.linalg.norm(r.x - xo) <= 1e-7 * np.linalg.norm(xo)
+
+
+def test_mixed_sizes_from_threads():
+    """Small items run beside the large ones of their call: from two threads,
+    call after call, each item's bits are those of a call of its kind alone."""
+    kinds = []
+    for dim, N, k in ((3, 18, 6), (2, 40, 30)):  # 5832 and 1600 rows
+        A = cmamd.gen_convdiff(dim, N, 1.0, seed=N)
+        s = cmamd.System("afiim", A, cmamd.afiim(A, 0.1))
+        kinds.append([(s, cmamd.csr_mv_host(A, cmamd.gen_uniform(j, A.n)), None, 1e-8, 500) for j in range(k)])
+    want = [r.x for it in kinds for r in cmamd.batch_solve(it)]
+    mixed = kinds[0] + kinds[1]
+    bad = []
+
+    def loop():
+        for rep in range(6):
+            for q, r in enumerate(cmamd.batch_solve(mixed)):
+                if r.info != 0 or not np.array_equal(r.x, want[q]):
+                    bad.append((rep, q, r.info))
+
+    th = [threading.Thread(target=loop) for _ in range(2)]
+    for t in th:
+        t.start()
+    for t in th:
+        t.join()
+    assert not bad, bad
