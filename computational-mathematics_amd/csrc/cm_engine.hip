@@ -1260,6 +1260,12 @@ struct RsRunner {
         (void)hipFree(args);
         if (out) (void)hipHostFree(out);
     }
+    // device bytes of a runner for up to nc columns, and those held
+    static size_t bytes_for(int nc)
+    {
+        return (size_t)nc * RS_SETS * RS_K * RS_WGS * sizeof(double) + sizeof(RsCtl) + sizeof(RsTable<T, VA, VF>);
+    }
+    size_t bytes() const { return ctl ? bytes_for(slot_cols) : 0; }
     static int cus(int *dev)
     {
         int c = 0;
@@ -1510,7 +1516,7 @@ struct Krylov {
     {
         return A.bytes() + G.bytes() + H.bytes() + GT.bytes() + L.bytes() + U.bytes() +
                15 * (size_t)n * sizeof(T) + (size_t)std::max(A.nblk, MAX_RED_BLOCKS) * 4 * sizeof(double) +
-               (size_t)trace_cap_dev * sizeof(double);
+               (size_t)trace_cap_dev * sizeof(double) + rs.bytes();
     }
 
     bool uses_gh() const { return variant != 2 || mode == 'E' || mode == 'C'; }
@@ -2396,7 +2402,7 @@ struct BlockKrylov {
                std::max(slots, (size_t)MAX_RED_BLOCKS) * 4 * KB * sizeof(double) + 3 * (size_t)n * sizeof(int) +
                racc * sizeof(T);
     }
-    size_t bytes() const { return bytes_for(n, partial_slots, racc_cap); }
+    size_t bytes() const { return bytes_for(n, partial_slots, racc_cap) + rs.bytes(); }
 
     template <class KR>
     int create(const KR &k, hipStream_t strm)
@@ -3097,7 +3103,8 @@ static size_t block_bytes_estimate(const K64 &k64, int kb, int bits)
                3 * (size_t)n * sizeof(int) + kb * sizeof(SolveState) + sizeof(BlockFlags) + racc * vsz;
     };
     size_t b = one(sizeof(double)) + (size_t)n * kb * sizeof(double);
-    if (bits == 32 || bits == 16) b += one(sizeof(float));
+    if (bits == 32 || bits == 16) b += one(sizeof(float)) + RsRunner<float, float, float>::bytes_for(kb);
+    else b += RsRunner<double, double, double>::bytes_for(kb);
     return b;
 }
 
