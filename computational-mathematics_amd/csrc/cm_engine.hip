@@ -3602,10 +3602,13 @@ int pd_take(T **h, const T *d, size_t count, hipStream_t s)
     return copy_d2h(*h, d, count, s);
 }
 
-// Device buffers of one construction, freed on every exit.
-// Cut from a few chunks of doubling size: an allocation and its release cost
-// some 0.3 ms each, 12 ms of a 64^3 construction with one per buffer.
+// Device buffers of one construction, freed on every exit.  Small ones are cut
+// from a few chunks of doubling size up to CHUNK_MAX: an allocation and its
+// release cost some 0.3 ms each, 12 ms of a 64^3 construction with one per
+// buffer.  Those of half of CHUNK_MAX and more are allocations of their own, so
+// no more than some CHUNK_MAX is held beyond what is asked for.
 struct PdBuffers {
+    static constexpr size_t CHUNK_MAX = (size_t)256 << 20;
     std::vector<void *> held;
     hipStream_t stream = nullptr;
     char *at = nullptr;
@@ -3614,8 +3617,15 @@ struct PdBuffers {
     int alloc(T **d, size_t count)
     {
         const size_t bytes = (std::max<size_t>(count, 1) * sizeof(T) + 255) / 256 * 256;
+        if (bytes > left && bytes >= CHUNK_MAX / 2) {
+            char *own;
+            CM_TRY(dev_alloc(&own, bytes));
+            held.push_back(own);
+            *d = reinterpret_cast<T *>(own);
+            return CM_OK;
+        }
         if (bytes > left) {
-            chunk = std::max(2 * chunk, bytes);
+            chunk = std::max(std::min(2 * chunk, CHUNK_MAX), bytes);
             at = nullptr;
             left = 0;
             CM_TRY(dev_alloc(&at, chunk));
