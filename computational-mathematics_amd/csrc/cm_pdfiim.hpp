@@ -489,11 +489,13 @@ __global__ __launch_bounds__(BS) void k_pd_rows(int n, const O *__restrict__ ofs
 }
 
 // ptr[c] = first place of a key >= c among the sorted keys, c = 0 .. n.
+// (Walks over entries count in 64 bits: the step past the last of some 2^31
+// would turn a 32-bit one negative.)
 __global__ __launch_bounds__(BS) void k_pd_bounds(int n, int nnz, const int *__restrict__ key, int *__restrict__ ptr)
 {
-    for (int k = blockIdx.x * BS + threadIdx.x; k <= nnz; k += gridDim.x * BS) {
+    for (long long k = (long long)blockIdx.x * BS + threadIdx.x; k <= nnz; k += (long long)gridDim.x * BS) {
         const int lo = k ? key[k - 1] + 1 : 0, hi = k < nnz ? key[k] : n;
-        for (int c = lo; c <= hi; c++) ptr[c] = k;
+        for (int c = lo; c <= hi; c++) ptr[c] = (int)k;
     }
 }
 
@@ -502,7 +504,7 @@ __global__ __launch_bounds__(BS) void k_pd_permute(int nnz, const int *__restric
                                                    const double *__restrict__ val, int *__restrict__ tidx,
                                                    double *__restrict__ tval)
 {
-    for (int q = blockIdx.x * BS + threadIdx.x; q < nnz; q += gridDim.x * BS) {
+    for (long long q = (long long)blockIdx.x * BS + threadIdx.x; q < nnz; q += (long long)gridDim.x * BS) {
         const int k = ent[q];
         tidx[q] = row[k];
         tval[q] = val[k];
