@@ -1734,7 +1734,7 @@ struct Krylov {
                 const long long waves = std::min<long long>(512, 5LL * m.nchunk / (2LL * std::max(1, m.nlev)) + 4);
                 const int g = (int)(TRSV_XCDS * ((waves + TRSV_BS / WAVE - 1) / (TRSV_BS / WAVE)));
                 k_trsv_flow<T, VF, LPR><<<g, TRSV_BS, 0, stream>>>(m.nchunk, m.rpc, m.crow, m.tcol, m.tval, m.rowscale,
-                                                                  bin, dscale, xout, trsv_ctl + q,
+                                                                  bin, dscale, xout, trsv_ctl + q, rs.control->spins,
                                                                   use_state ? st : nullptr, use_state ? st : nullptr);
             };
             switch (m.lpr) {
@@ -3864,7 +3864,14 @@ int cm_system_resident(cm_system h, int on, int spins, int join_us, long long *c
     RsControl &c = *h->sys.k64->rs.control;
     c.on = on != 0;
     c.skip = 0;
+    const int before = c.spins;
     c.spins = spins < 0 ? RS_SPINS : std::min(spins, RS_SPINS);
+    if (c.spins != before) {  // captured triangular solves carry the limit
+        CM_HIP(hipStreamSynchronize(h->sys.stream));
+        h->sys.k64->drop_graphs();
+        if (h->sys.k32) h->sys.k32->drop_graphs();
+        if (h->sys.k16) h->sys.k16->drop_graphs();
+    }
     c.join_ticks = join_us < 0 ? RS_JOIN_TICKS : std::min(100LL * join_us, RS_JOIN_TICKS);
     if (counts) {
         counts[0] = c.solved;

@@ -14,7 +14,7 @@
 // together and could not), and tickets are handed out in chunk order to waves
 // that are already running: the wave with the lowest unfinished chunk finds
 // all it reads, and every wait ends, with any number of waves.  A wait that
-// does not end within RS_SPINS looks is given up all the same: fail is set,
+// does not end within `spins` looks is given up all the same: fail is set,
 // everybody leaves, and the host reports an error.
 //
 // What bounds the solve is the chain of levels (about 240 and 440 in the
@@ -130,7 +130,7 @@ template <class T, class V, int LPR>
 __global__ __launch_bounds__(TRSV_BS) void k_trsv_flow(int chunks, int rpc, const int4 *__restrict__ crow,
                                                        const int *__restrict__ tcol, const V *__restrict__ tval,
                                                        const float *__restrict__ rowscale, const T *__restrict__ b,
-                                                       const T *__restrict__ dscale, T *x, TrsvCtl *c,
+                                                       const T *__restrict__ dscale, T *x, TrsvCtl *c, int spins,
                                                        const SolveState *st, SolveState *rep)
 {
     static_assert(LPR >= 1 && LPR <= WAVE && (LPR & (LPR - 1)) == 0, "lanes per row: a power of two");
@@ -187,8 +187,8 @@ __global__ __launch_bounds__(TRSV_BS) void k_trsv_flow(int chunks, int rpc, cons
 #pragma unroll
             for (int e = 0; e < P; e++) miss |= w[e] == B::MARK;
             if (!miss) break;
-            if (spin % 1024 == 0) {
-                if (spin >= RS_SPINS) __hip_atomic_store(&c->fail, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            if (spin % 1024 == 0 || spin >= spins) {
+                if (spin >= spins) __hip_atomic_store(&c->fail, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
                 if (__hip_atomic_load(&c->fail, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)) gone = true;
             }
             if (gone) break;

@@ -160,7 +160,8 @@ int cm_system_block_graphs(cm_system sys, int on);
  * default limits).  counts (or null) receives the right-hand sides so far
  * that resident launches solved, whose grid did not arrive, and in which a
  * wait was given up: the latter two took the launched passes from their
- * starting x. */
+ * starting x.  spins holds for the triangular solves' waits too, which end
+ * the solve or apply with CM_ERR_HIP. */
 int cm_system_resident(cm_system sys, int on, int spins, int join_us, long long counts[3]);
 /* Persistent batched solves: nitems right-hand sides of small resident
  * systems (item i: system systems[i], column B[i], initial guess and result
