@@ -292,12 +292,17 @@ static int copy_h2d(T *d, const T *h, size_t count, hipStream_t s)
 }
 
 // Device to host (pageable), large arrays through pinned chunks; small ones
-// are only enqueued.
+// are only enqueued, and those of a stream on another device than the current
+// one, on which the chunks' events could not be recorded.
 template <class T>
 static int copy_d2h(T *h, const T *d, size_t count, hipStream_t s)
 {
     const size_t bytes = count * sizeof(T);
-    if (bytes >= Stager::MIN_BYTES) return Stager::get().download(h, d, bytes, s);
+    int cur = -1;
+    hipDevice_t of = -1;
+    if (bytes >= Stager::MIN_BYTES && hipGetDevice(&cur) == hipSuccess && hipStreamGetDevice(s, &of) == hipSuccess &&
+        of == cur)
+        return Stager::get().download(h, d, bytes, s);
     if (bytes) CM_HIP(hipMemcpyAsync(h, d, bytes, hipMemcpyDeviceToHost, s));
     return CM_OK;
 }
@@ -1387,7 +1392,7 @@ struct RsRunner {
     // all of them did; else x is as it was in those that did not (a.save; on a
     // zero start it need not be).
     // A grid that does not arrive in RS_JOIN_TICKS leaves and is tried again,
-    // RS_TRIES times with pauses: by then kernels of some 0.3 s have ended.
+    // RS_TRIES times with pauses: by then kernels of some 0.2 s have ended.
     int run(RsArgs<T, VA, VF> &a, const DevCsr<VA> &A, const DevCsr<VF> &H, const DevCsr<VF> &G, const RsPlan &p,
             hipStream_t stream, bool &ran)
     {

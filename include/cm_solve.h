@@ -152,7 +152,7 @@ int cm_system_block_graphs(cm_system sys, int on);
  * suit it (on, the default) or never (off: launched passes).  Which of the
  * two a solve takes, and in what order it sums, depends on the system and the
  * block width alone: grids of concurrent solves wait for their turn.  Only
- * when other work on the device keeps a grid from starting for some 0.3 s
+ * when other work on the device keeps a grid from starting for some 0.2 s
  * does the solve (and the next 16) take the launched passes, whose sums
  * differ by rounding.  spins and
  * join_us lower the looks of one wait and the time a grid has to arrive
