@@ -746,7 +746,7 @@ def _leg_args(args, name):
 
 def _leg_summary(out, wall_s):
     """The figures of a workload's full line that a compact leg reports."""
-    keep = ("value", "unit", "ms_per_step", "steps", "dtype", "latency_ms", "queue_ms", "service_ms",
+    keep = ("value", "unit", "ms_per_step", "steps", "dtype", "solve", "latency_ms", "queue_ms", "service_ms",
             "iterations", "info", "true_rel_residual", "true_rel_residual_max", "forward_error_vs_xstar",
             "forward_error_vs_xstar_max", "rel_error_vs_oracle", "rel_error_vs_oracle_column0",
             "rel_error_vs_fp64_solution_max", "outer_steps", "inner_passes", "fp64_one_at_a_time", "fp64_block",
@@ -807,9 +807,11 @@ def bench_single(args, w):
             sys_.enable_mixed(16)
         tuned = sys_.autotune(reps=10)
     sys_.set_rhs(b)
-    for _ in range(args.warmup):
+    c0 = sys_.resident()[0]
+    for _ in range(max(1, args.warmup)):
         sys_.set_x(None)
         sys_.solve(tol=w["tol"], nmax=w["nmax"])
+    resident = sys_.resident()[0] > c0  # whole solves in one launch
     # per-kernel breakdown: two extra solves with every launch bracketed
     sys_.profile(True)
     for _ in range(2):
@@ -822,10 +824,11 @@ def bench_single(args, w):
     # SAMPLE_PASSES passes of each solve (launched kernel by kernel); the other passes replay from
     # the captured graphs, as in an unprofiled solve.  A dominant category of many launches per pass
     # (thousands of small ones, say) is timed in separate solves
-    # instead: events around each of its launches would slow the timed solves themselves.
+    # instead: events around each of its launches would slow the timed solves themselves.  So it is
+    # where solves run in one resident launch, which profiling would replace by launched passes.
     profiled_passes = max(1, stats["A"][0] // 2)  # passes of the two profiled solves (two A products each)
     kernel_timing = args.kernel_timing
-    if stats[dom][0] / profiled_passes > DOM_LAUNCHES_PER_PASS_MAX:
+    if resident or stats[dom][0] / profiled_passes > DOM_LAUNCHES_PER_PASS_MAX:
         kernel_timing = "separate"
     sys_.profile(kernel_timing == "timed-region", cats=(dom,), sample=SAMPLE_PASSES)
     lat = []
@@ -950,6 +953,7 @@ def bench_single(args, w):
                    "tol": w["tol"], "nmax": w["nmax"], "symmetric": sym},
         "latency_ms": {"p50": round(1e3 * float(np.percentile(lat, 50)), 3),
                        "p99": round(1e3 * float(np.percentile(lat, 99)), 3)},
+        "solve": "one resident launch" if resident else "launched passes",
         "iterations": int(np.median(iters)), "info": info, "resval": rv, "true_rel_residual": true_res,
         "forward_error_vs_xstar": fwd_err,
         "mixed_precision": mixed, "autotune_tiles": tuned,
@@ -965,7 +969,8 @@ def bench_single(args, w):
             f"first {SAMPLE_PASSES} passes of each solve (the rest replay from hipGraphs)"
             if kernel_timing == "timed-region" else
             "roofline from 3 solves after the timed region with the dominant kernel's launches bracketed "
-            "(the timed solves carry no events)"),
+            "(the timed solves carry no events)") + (
+            "; the tables are those of launched passes, the timed solves run in one launch" if resident else ""),
     }
     if not args.no_cpu:
         out["cpu_baseline"], x_or = cpu_baseline(w, A, b, F, args.cpu_seconds)
