@@ -173,9 +173,10 @@ int cm_system_resident(cm_system sys, int on, int spins, int join_us, long long 
  * while its true residual is above tol (at most 4 cycles, NMAX passes in
  * total); 0 is the reference loop.  Apply mode E; per-item resval, iter,
  * info as in cm_system_solve.  Suited to systems whose solve is launch-bound
- * (up to some 10^4-10^5 rows); up to 4096 rows they stay in LDS and
- * registers, above that work vectors take 9 n doubles per resident
- * workgroup. */
+ * (up to some 10^4-10^5 rows); up to 4096 rows (of 80 to 170 entries on the
+ * mean at most) they stay in LDS and registers, in a kernel of their own that
+ * runs beside the other one; in that work vectors take 9 n doubles per
+ * resident workgroup. */
 int cm_batch_solve(int nitems, const cm_system *systems, const double *const *B, double *const *X,
                    const double *tol, const int *NMAX, int restart_true, double *resval, int *iter, int *info);
 
